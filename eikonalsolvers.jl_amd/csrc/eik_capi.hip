@@ -36,6 +36,8 @@ void set_tiles(InstDev& I, int nd) {
         I.t[d] = d < nd ? (I.n[d] + fe - 1) / fe : 1;
         I.at[d] = d < nd ? (I.n[d] + ae - 1) / ae : 1;
     }
+    I.rbx = 1.0 / (double)I.t[0];
+    I.rby = 1.0 / (double)I.t[1];
 }
 
 static inline double gcoord(const eik_grid& g, int d, int64_t i) {

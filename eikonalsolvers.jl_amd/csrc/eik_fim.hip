@@ -64,20 +64,6 @@ __device__ __forceinline__ int find_inst(const InstDev* __restrict__ inst, int n
     return lo;
 }
 
-// Minimum of v over the 64 lanes of the wave, wave-uniform; every lane must be active.  Quad
-// swaps and row rotations (DPP) reduce each row of 16 lanes, and the four row minima are read out
-// to scalar registers.  (An LDS atomicMin per lane instead compiles to a loop over the active
-// lanes, several scalar instructions per lane.)
-__device__ __forceinline__ unsigned wave_min_u32(unsigned v) {
-    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
-    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xF, 0xF, true));  // row_ror:4
-    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true));  // row_ror:8
-    const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0), b = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
-    const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)v, 32), d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
-    return min(min(a, b), min(c, d));
-}
-
 template <typename T>
 __device__ __forceinline__ bool is_fixed(T raw) {
     return signbit(raw);
@@ -814,12 +800,6 @@ __global__ void k_fill_u32(unsigned* __restrict__ p, int64_t n, unsigned v) {
     if (i < n) p[i] = v;
 }
 
-template <typename T>
-__global__ void k_fill(T* __restrict__ p, int64_t n, T v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 __global__ void k_slowness(const double* __restrict__ vel, double* __restrict__ s64, float* __restrict__ s32,
                            int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -835,8 +815,8 @@ __global__ void k_slowness(const double* __restrict__ vel, double* __restrict__ 
 // boxes (vel = the nearest-neighbour fine velocity, read through the box's map).
 template <typename T>
 __global__ void k_corners(const CornerDev* __restrict__ cs, int ncs, const InstDev* __restrict__ inst,
-                          T* __restrict__ ttpool, const FineDev* __restrict__ fine, unsigned* __restrict__ flags,
-                          unsigned* __restrict__ pend, int nd, int kind) {
+                          T* __restrict__ ttpool, uint8_t* __restrict__ dpool, const FineDev* __restrict__ fine,
+                          unsigned* __restrict__ flags, unsigned* __restrict__ pend, int nd, int kind) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= ncs) return;
     const CornerDev C = cs[q];
@@ -854,7 +834,10 @@ __global__ void k_corners(const CornerDev* __restrict__ cs, int ncs, const InstD
     }
     const double dist = C.dist;
     ttpool[I.tt_off + l] = -(T)(dist / v);
-    seed_tiles_fwd(I, nd, g, flags, pend, dist / v);
+    if (dpool)
+        dpool[I.tt_off + l] = (uint8_t)kInitDepth;
+    else
+        seed_tiles_fwd(I, nd, g, flags, pend, dist / v);
 }
 
 // nearest-neighbour fine slowness of every refined box (createfinegrid, eikmainfwd.jl:1035-1056)
@@ -889,8 +872,8 @@ __global__ void k_fine_setup(const FineDev* __restrict__ fine, int nfine, const 
 template <typename T>
 __global__ void __launch_bounds__(256) k_transfer(const FineDev* __restrict__ fine, InstDev* __restrict__ finst,
                                                   TTPools fp, const InstDev* __restrict__ cinst, T* __restrict__ ttc,
-                                                  unsigned* __restrict__ cflags, unsigned* __restrict__ cpend,
-                                                  int* __restrict__ ntransfer, SrcPt* __restrict__ xlist, int cap,
+                                                  uint8_t* __restrict__ dpool, unsigned* __restrict__ cflags,
+                                                  unsigned* __restrict__ cpend, int* __restrict__ ntransfer, SrcPt* __restrict__ xlist, int cap,
                                                   int nd) {
     const int f = blockIdx.x;
     const FineDev F = fine[f];
@@ -972,7 +955,10 @@ __global__ void __launch_bounds__(256) k_transfer(const FineDev* __restrict__ fi
                 const int cg[3] = {F.i1c[0] + wx, F.i1c[1] + wy, F.i1c[2] + wz};
                 const int64_t lc = cg[0] + (int64_t)C.n[0] * (cg[1] + (int64_t)C.n[1] * cg[2]);
                 ttc[C.tt_off + lc] = -(T)t;
-                seed_tiles_fwd(C, nd, cg, cflags, cpend, t);
+                if (dpool)
+                    dpool[C.tt_off + lc] = (uint8_t)kInitDepth;
+                else
+                    seed_tiles_fwd(C, nd, cg, cflags, cpend, t);
                 if (cnt < cap) xlist[(int64_t)f * cap + cnt] = SrcPt{F.cinst, (int32_t)lf, lc};
                 cnt++;
             }
@@ -1016,7 +1002,7 @@ static unsigned claim_chunk() {
 }
 
 // Relative size below which an FP32 change wakes no other node (EIK_F32_SETTLE overrides).
-static double f32_settle() {
+double f32_settle() {
     static const double v = [] {
         const char* e = getenv("EIK_F32_SETTLE");
         return e ? atof(e) : 0.0;
@@ -1026,7 +1012,7 @@ static double f32_settle() {
 
 // Relative size below which a mixed-precision change wakes no other node (EIK_MIX_SETTLE overrides;
 // default 0: every change propagates and the mixed solve replays the mixed heap FMM exactly).
-static double mix_settle() {
+double mix_settle() {
     static const double v = [] {
         const char* e = getenv("EIK_MIX_SETTLE");
         return e ? atof(e) : 0.0;
@@ -1282,6 +1268,14 @@ static double corner_dist(const InstDev& I, int nd, int kind, const int* ijk, co
     return distance2points(kind, nd, xyz, src);
 }
 
+// The whole solve again, by the tile solver (a march whose lists were too short).
+static int solve_with_tiles(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
+    ctx->tiles_only = true;
+    const int rc = forward_solve(ctx, G, prec, P);
+    ctx->tiles_only = false;
+    return rc;
+}
+
 int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
     const eik_model* M0 = G[0].M;
     const int nd = M0->g.ndim;
@@ -1322,10 +1316,12 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
 
     // coarse instances: one grid per source, sharing its model's slowness
     std::vector<InstDev> cinst(nsrc);
-    int64_t ntiles_c = 0, antiles_c = 0, totN = 0;
+    int64_t ntiles_c = 0, antiles_c = 0, totN = 0, stiles_c = 0, most_c = 0;
+    std::vector<int> owners_c;  // the first instance of every model
     {
         int64_t s = 0;
-        for (size_t k = 0; k < G.size(); k++)
+        for (size_t k = 0; k < G.size(); k++) {
+            owners_c.push_back((int)s);
             for (int64_t j = 0; j < G[k].S->nsrc; j++, s++) {
                 const eik_model* M = G[k].M;
                 InstDev& I = cinst[s];
@@ -1336,6 +1332,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                 set_tiles(I, nd);
                 I.tt_off = totN;
                 I.s_off = soff[k];
+                I.ms_off = stiles_c * 64;
                 I.tile_base = ntiles_c;
                 I.atile_base = antiles_c;
                 set_band(I, nd, prec, M->smean);
@@ -1356,8 +1353,11 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                 }
                 totN += M->N;
                 ntiles_c += (int64_t)I.t[0] * I.t[1] * I.t[2];
+                most_c = std::max(most_c, (int64_t)I.t[0] * I.t[1] * I.t[2]);
                 antiles_c += (int64_t)I.at[0] * I.at[1] * I.at[2];
             }
+            stiles_c += (int64_t)cinst[s - 1].t[0] * cinst[s - 1].t[1] * cinst[s - 1].t[2];
+        }
     }
     DevBuf& ttc = ctx->buf("tt_coarse");
     DevBuf& kc = ctx->buf("key_K");
@@ -1367,14 +1367,6 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
         dc.ensure((size_t)totN))
         return ctx->fail(EIK_ENOMEM, "out of device memory (traveltime grids)");
     CK(hipMemsetAsync(dc.p, 0, (size_t)totN, st));
-    // key pools start as an unreached node's key (+inf, -inf)
-    if (f32) {
-        k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)kc.p, totN, EIK_INFF);
-        k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)sc.p, totN, -EIK_INFF);
-    } else {
-        k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)kc.p, totN, EIK_INF);
-        k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)sc.p, totN, -EIK_INF);
-    }
     const TTPools cpools{ttc.p, kc.p, sc.p, (uint8_t*)dc.p};
     DevBuf& dci = ctx->buf("inst_coarse");
     if (dci.ensure(cinst.size() * sizeof(InstDev))) return ctx->fail(EIK_ENOMEM, "out of device memory");
@@ -1383,7 +1375,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     int64_t maxt = ntiles_c, maxat = antiles_c;
     std::vector<FineDev> fine;
     std::vector<InstDev> finst;
-    int64_t ntiles_f = 0, antiles_f = 0, nfine_pts = 0;
+    int64_t ntiles_f = 0, antiles_f = 0, nfine_pts = 0, most_f = 0;
     if (P->refinearoundsrc) {
         fine.resize(nsrc);
         finst.resize(nsrc);
@@ -1394,10 +1386,12 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
             finst[s].tt_off = nfine_pts;
             finst[s].s_off = nfine_pts;
             finst[s].tile_base = ntiles_f;
+            finst[s].ms_off = ntiles_f * 64;
             finst[s].atile_base = antiles_f;
             set_band(finst[s], nd, EIK_PREC_FP64, smod[s]->smean);  // refined boxes solve in FP64
             nfine_pts += (int64_t)finst[s].n[0] * finst[s].n[1] * finst[s].n[2];
             ntiles_f += (int64_t)finst[s].t[0] * finst[s].t[1] * finst[s].t[2];
+            most_f = std::max(most_f, (int64_t)finst[s].t[0] * finst[s].t[1] * finst[s].t[2]);
             antiles_f += (int64_t)finst[s].at[0] * finst[s].at[1] * finst[s].at[2];
         }
         maxt = std::max(maxt, ntiles_f);
@@ -1418,6 +1412,25 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
             for (int64_t s = 0; s < nsrc; s++) finst[s].sinth = (const double*)ft.p + off[s];
         }
     }
+    // Ordered marching where its buffers fit beside the pools; the tile solver, which needs about 50
+    // bytes a node less, otherwise (a no-allocation call near its limit, a device that is nearly
+    // full, a server near its budget).
+    MarchSize msz[2] = {march_size(nd, kind, prec, ntiles_c, stiles_c, most_c, (int)nsrc, (int)G.size()),
+                        march_size(nd, kind, EIK_PREC_FP64, ntiles_f, ntiles_f, most_f, (int)nsrc, (int)nsrc)};
+    const bool fits = march_reserve(ctx, msz, P->refinearoundsrc ? 2 : 1, (int)nsrc);
+    const bool march = fits && msz[0].mode != kMarchNone;                           // the grids
+    const bool march_f = fits && P->refinearoundsrc && msz[1].mode != kMarchNone;   // the refined boxes
+    const bool any_march = march || march_f, any_tiles = !march || (P->refinearoundsrc && !march_f);
+    if (!march) {
+        // the tile solver's key pools start as an unreached node's key (+inf, -inf)
+        if (f32) {
+            k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)kc.p, totN, EIK_INFF);
+            k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)sc.p, totN, -EIK_INFF);
+        } else {
+            k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)kc.p, totN, EIK_INF);
+            k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)sc.p, totN, -EIK_INF);
+        }
+    }
     DevBuf& aflags = ctx->buf("fim_flags");  // adjoint rounds, one byte per adjoint tile
     DevBuf& apend = ctx->buf("adj_pend");    // and its pending traveltime
     if (aflags.ensure((size_t)maxat) || apend.ensure((size_t)maxat * sizeof(unsigned)))
@@ -1425,19 +1438,40 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     CK(hipMemsetAsync(aflags.p, 0, (size_t)maxat, st));
     CK(hipMemsetAsync(apend.p, 0, (size_t)maxat * sizeof(unsigned), st));
     DevBuf& flags = ctx->buf("fim_tflags");
-    if (flags.ensure((size_t)maxt * sizeof(unsigned))) return ctx->fail(EIK_ENOMEM, "out of device memory (tile flags)");
-    CK(hipMemsetAsync(flags.p, 0, (size_t)maxt * sizeof(unsigned), st));
     DevBuf& pend = ctx->buf("fim_pend");
-    if (pend.ensure((size_t)maxt * sizeof(unsigned))) return ctx->fail(EIK_ENOMEM, "out of device memory (tile flags)");
-    k_fill_u32<<<nblocks(maxt, 256), 256, 0, st>>>((unsigned*)pend.p, maxt, 0x7f800000u);
+    if (any_tiles) {
+        if (flags.ensure((size_t)maxt * sizeof(unsigned)) || pend.ensure((size_t)maxt * sizeof(unsigned)))
+            return ctx->fail(EIK_ENOMEM, "out of device memory (tile flags)");
+        CK(hipMemsetAsync(flags.p, 0, (size_t)maxt * sizeof(unsigned), st));
+        k_fill_u32<<<nblocks(maxt, 256), 256, 0, st>>>((unsigned*)pend.p, maxt, 0x7f800000u);
+    }
 
-    // coarse grids start at +inf
-    if (prec != EIK_PREC_FP32)
+    // coarse grids start at +inf (a march writes every node at its end)
+    if (march) {
+    } else if (prec != EIK_PREC_FP32)
         k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)ttc.p, totN, EIK_INF);
     else
         k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)ttc.p, totN, EIK_INFF);
 
     std::vector<CornerDev> corners;
+    // the march's init nodes: the source-box corners, or the points transferred from the refined box
+    constexpr int kCorn = 8;
+    std::vector<SrcPt> seedpt(any_march ? (size_t)nsrc * kCorn : 0);
+    std::vector<int> nseed(any_march ? (size_t)nsrc : 0);
+    DevBuf &dsp = ctx->buf("march_seed"), &dns = ctx->buf("march_nseed");
+    std::vector<int> owners = owners_c;  // then every refined box, which has its own slowness
+    if (any_march) {
+        for (int64_t s = 0; s < nsrc; s++) owners.push_back((int)s);
+        if (dsp.ensure(seedpt.size() * sizeof(SrcPt)) || dns.ensure((nseed.size() + owners.size()) * sizeof(int)))
+            return ctx->fail(EIK_ENOMEM, "out of device memory");
+        CK(hipMemcpyAsync((int*)dns.p + nsrc, owners.data(), owners.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        msz[0].owners = (const int*)dns.p + nsrc;
+        msz[1].owners = msz[0].owners + owners_c.size();
+    }
+    auto add_seed = [&](int64_t s, const InstDev& I, const int* g) {
+        if (any_march) seedpt[(size_t)(s * kCorn + nseed[s]++)] = SrcPt{(int32_t)s, -1, g[0] + (int64_t)I.n[0] * (g[1] + (int64_t)I.n[1] * g[2])};
+    };
+    MarchSeeds seeds{(const SrcPt*)dsp.p, kCorn, (const int*)dns.p, march_ctl(cinst)};
     if (P->refinearoundsrc) {
         DevBuf& dfi = ctx->buf("inst_fine");
         DevBuf& dfd = ctx->buf("fine_desc");
@@ -1452,8 +1486,10 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
             df.ensure((size_t)nfine_pts))
             return ctx->fail(EIK_ENOMEM, "out of device memory (refined grids)");
         CK(hipMemsetAsync(df.p, 0, (size_t)nfine_pts, st));
-        k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)kf.p, nfine_pts, EIK_INF);
-        k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)sf.p, nfine_pts, -EIK_INF);
+        if (!march_f) {
+            k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)kf.p, nfine_pts, EIK_INF);
+            k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)sf.p, nfine_pts, -EIK_INF);
+        }
         const TTPools fpools{ttf.p, kf.p, sf.p, (uint8_t*)df.p};
         CK(hipMemcpyAsync(dfi.p, finst.data(), finst.size() * sizeof(InstDev), hipMemcpyHostToDevice, st));
         CK(hipMemcpyAsync(dfd.p, fine.data(), fine.size() * sizeof(FineDev), hipMemcpyHostToDevice, st));
@@ -1469,21 +1505,29 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                 C.dist = corner_dist(finst[s], nd, kind, C.ijk, C.src);
                 C.vel = smod[s]->d_vel;
                 corners.push_back(C);
+                add_seed(s, finst[s], C.ijk);
             }
         }
         DevBuf& dcs = ctx->buf("corners");
         if (dcs.ensure(corners.size() * sizeof(CornerDev))) return ctx->fail(EIK_ENOMEM, "out of device memory");
         CK(hipMemcpyAsync(dcs.p, corners.data(), corners.size() * sizeof(CornerDev), hipMemcpyHostToDevice, st));
+        if (any_march) {
+            CK(hipMemcpyAsync(dsp.p, seedpt.data(), seedpt.size() * sizeof(SrcPt), hipMemcpyHostToDevice, st));
+            CK(hipMemcpyAsync(dns.p, nseed.data(), nseed.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        }
         k_corners<double><<<nblocks((int64_t)corners.size(), 64), 64, 0, st>>>(
             (const CornerDev*)dcs.p, (int)corners.size(), (const InstDev*)dfi.p, (double*)ttf.p,
-            (const FineDev*)dfd.p, (unsigned*)flags.p, (unsigned*)pend.p, nd, kind);
+            march_f ? (uint8_t*)df.p : nullptr, (const FineDev*)dfd.p, (unsigned*)flags.p, (unsigned*)pend.p, nd, kind);
         CK(hipGetLastError());
         tm.mark();
         FimStats fst{};
         ctx->span_fine = true;
-        int rc = fim_run(ctx, nd, EIK_PREC_FP64, kind, (const InstDev*)dfi.p, (int)nsrc, ntiles_f, fpools, slf.p,
-                         P->fast == 0, false, &fst);
+        int rc = march_f ? march_run(ctx, nd, EIK_PREC_FP64, kind, (const InstDev*)dfi.p, (int)nsrc, msz[1], fpools, slf.p, seeds,
+                                   P->fast == 0, false, &fst)
+                       : fim_run(ctx, nd, EIK_PREC_FP64, kind, (const InstDev*)dfi.p, (int)nsrc, ntiles_f, fpools, slf.p,
+                                 P->fast == 0, false, &fst);
         ctx->span_fine = false;
+        if (rc == kMarchOverflow) return solve_with_tiles(ctx, G, prec, P);
         if (rc) return rc;
         ctx->stats[1] = tm.mark();
         ctx->stats[14] = fst.kernel_ms;
@@ -1502,13 +1546,18 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
             return ctx->fail(EIK_ENOMEM, "out of device memory");
         if (prec != EIK_PREC_FP32)
             k_transfer<double><<<(unsigned)nsrc, 256, 0, st>>>((const FineDev*)dfd.p, (InstDev*)dfi.p, fpools,
-                                                              (const InstDev*)dci.p, (double*)ttc.p, (unsigned*)flags.p,
+                                                              (const InstDev*)dci.p, (double*)ttc.p,
+                                                              march ? (uint8_t*)dc.p : nullptr, (unsigned*)flags.p,
                                                               (unsigned*)pend.p, (int*)ntr.p, (SrcPt*)xl.p, cap, nd);
         else
             k_transfer<float><<<(unsigned)nsrc, 256, 0, st>>>((const FineDev*)dfd.p, (InstDev*)dfi.p, fpools,
-                                                             (const InstDev*)dci.p, (float*)ttc.p, (unsigned*)flags.p,
+                                                             (const InstDev*)dci.p, (float*)ttc.p,
+                                                              march ? (uint8_t*)dc.p : nullptr, (unsigned*)flags.p,
                                                              (unsigned*)pend.p, (int*)ntr.p, (SrcPt*)xl.p, cap, nd);
         CK(hipGetLastError());
+        seeds.seeds = (const SrcPt*)xl.p;
+        seeds.cap = cap;
+        seeds.nseed = (const int*)ntr.p;
     } else {
         for (int64_t s = 0; s < nsrc; s++) {
             int corn[8][3];
@@ -1521,18 +1570,23 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                 C.dist = corner_dist(cinst[s], nd, kind, C.ijk, C.src);
                 C.vel = smod[s]->d_vel;
                 corners.push_back(C);
+                add_seed(s, cinst[s], C.ijk);
             }
         }
         DevBuf& dcs = ctx->buf("corners");
         if (dcs.ensure(corners.size() * sizeof(CornerDev))) return ctx->fail(EIK_ENOMEM, "out of device memory");
         CK(hipMemcpyAsync(dcs.p, corners.data(), corners.size() * sizeof(CornerDev), hipMemcpyHostToDevice, st));
+        if (any_march) {
+            CK(hipMemcpyAsync(dsp.p, seedpt.data(), seedpt.size() * sizeof(SrcPt), hipMemcpyHostToDevice, st));
+            CK(hipMemcpyAsync(dns.p, nseed.data(), nseed.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        }
         if (prec != EIK_PREC_FP32)
             k_corners<double><<<nblocks((int64_t)corners.size(), 64), 64, 0, st>>>(
-                (const CornerDev*)dcs.p, (int)corners.size(), (const InstDev*)dci.p, (double*)ttc.p, nullptr,
+                (const CornerDev*)dcs.p, (int)corners.size(), (const InstDev*)dci.p, (double*)ttc.p, march ? (uint8_t*)dc.p : nullptr, nullptr,
                 (unsigned*)flags.p, (unsigned*)pend.p, nd, kind);
         else
             k_corners<float><<<nblocks((int64_t)corners.size(), 64), 64, 0, st>>>(
-                (const CornerDev*)dcs.p, (int)corners.size(), (const InstDev*)dci.p, (float*)ttc.p, nullptr,
+                (const CornerDev*)dcs.p, (int)corners.size(), (const InstDev*)dci.p, (float*)ttc.p, march ? (uint8_t*)dc.p : nullptr, nullptr,
                 (unsigned*)flags.p, (unsigned*)pend.p, nd, kind);
         CK(hipGetLastError());
         tm.mark();
@@ -1540,8 +1594,11 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     FimStats cst{};
     // unrefined mixed solves give their instances an FP64 region around the source (above)
     const bool near = prec == EIK_PREC_MIXED && !P->refinearoundsrc;
-    int rc = fim_run(ctx, nd, prec, kind, (const InstDev*)dci.p, (int)nsrc, ntiles_c, cpools, slow, P->fast == 0,
-                     near, &cst);
+    int rc = march ? march_run(ctx, nd, prec, kind, (const InstDev*)dci.p, (int)nsrc, msz[0], cpools, slow, seeds, P->fast == 0,
+                               near, &cst)
+                   : fim_run(ctx, nd, prec, kind, (const InstDev*)dci.p, (int)nsrc, ntiles_c, cpools, slow, P->fast == 0,
+                             near, &cst);
+    if (rc == kMarchOverflow) return solve_with_tiles(ctx, G, prec, P);
     if (rc) return rc;
     ctx->stats[2] = tm.mark();
     ctx->stats[4] = cst.activations;

@@ -45,6 +45,8 @@ struct InstDev {
     double band;         // band scheduler: tiles within this traveltime of the lowest pending one run
     double nband;        // the same for the nodes updated inside a tile
     double aband;        // adjoint rounds: tiles within this traveltime of the highest pending one run
+    double rbx, rby;     // 1 / t[0], 1 / t[1]
+    int64_t ms_off;      // element offset of its slowness in the march's bricked slowness
     // mixed precision: nodes inside [xlo, xhi] (per axis) use the FP64 stencil (the near-source
     // region of an unrefined solve); empty when xlo > xhi
     int32_t xlo[3], xhi[3];
@@ -214,6 +216,20 @@ __device__ __forceinline__ void node_spacing(const InstDev& I, const int* g, T* 
     }
 }
 
+// Minimum of v over the 64 lanes of the wave, wave-uniform; every lane must be active.  Quad
+// swaps and row rotations (DPP) reduce each row of 16 lanes, and the four row minima are read out
+// to scalar registers.  (An LDS atomicMin per lane instead compiles to a loop over the active
+// lanes, several scalar instructions per lane.)
+__device__ __forceinline__ unsigned wave_min_u32(unsigned v) {
+    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
+    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true));   // quad_perm [2,3,0,1]
+    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x124, 0xF, 0xF, true));  // row_ror:4
+    v = min(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true));  // row_ror:8
+    const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0), b = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
+    const unsigned c = (unsigned)__builtin_amdgcn_readlane((int)v, 32), d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(a, b), min(c, d));
+}
+
 // Receiver interpolation on a traveltime grid (|value| strips the init-node sign).
 // bilinear_interp (eikforward2D.jl:17-87); trilinear_interp (eikforward3D.jl:17-140) keeps the
 // reference's weight xd*(1-yd)*(1-zd) for corner f101 so picks and gradients stay consistent
@@ -303,6 +319,7 @@ struct Arena {
     char* base = nullptr;
     size_t cap = 0;
     size_t used = 0;
+    size_t spare = 0;  // bytes beyond the call's bound, for buffers it can do without
     void* carve(size_t n) {
         const size_t at = (used + 255) & ~(size_t)255;
         if (!base || at > cap || n > cap - at) return nullptr;
@@ -383,6 +400,8 @@ struct eik_ctx {
     eik_ctx* owner = nullptr;  // set on a peer: the context it belongs to (whose tbase it shares)
     bool split = true;         // large calls may split their sources with the peer
     bool in_split = false;     // the current call is split (set on the context and its peer)
+    int64_t march_limit = -1;  // bytes the march's buffers may grow by in this call (-1: no limit)
+    bool tiles_only = false;   // the tile solver instead of a march (see forward_solve)
     int xcap = 1;  // capacity per source of the transferred-point list
     std::mutex mu;
     // arena mode (the no-allocation entry point): buffers are carved from this block instead
@@ -534,6 +553,11 @@ int gradient_solve(eik_ctx* ctx, eik_model* M, const SourceSet& S, const eik_par
                    const double* pickobs, const double* stdobs, double* gradvel, double* gradsrc, double* misf);
 // fill kernel (eik_fim.hip), also used by the adjoint rounds
 __global__ void k_fill_u32(unsigned* __restrict__ p, int64_t n, unsigned v);
+template <typename T>
+__global__ void k_fill(T* __restrict__ p, int64_t n, T v) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+}
 struct FimStats {
     int64_t rounds = 0;        // solver rounds (one launch each)
     double activations = 0;    // tile activations (blocks launched)
@@ -553,6 +577,42 @@ struct TTPools {
     void* s;
     uint8_t* d;
 };
+// Ordered marching (eik_march.hip).  Depth byte of an init node while a march runs; the init nodes of
+// every instance (cap entries each, `node` used); the settling stages and the limit, in rounds.
+constexpr int kInitDepth = 0xff;
+struct MarchCtl {
+    unsigned max_rounds, settle_round, settle_step;
+    double settle_tol;
+};
+struct MarchSeeds {
+    const SrcPt* seeds;
+    int cap;
+    const int* nseed;
+    MarchCtl ctl;
+};
+// What a march works on: bricks (forward tiles) of all instances, of their slowness grids (one per
+// model), and of the largest instance; the instances that own a slowness grid (device).
+struct MarchSize {
+    int64_t ntiles, stiles, most;
+    size_t esz;
+    const int* owners;
+    int nowners;
+    int mode;  // kMarch*
+};
+// kMarchNone: the tile solver; kMarchGroup: one workgroup per instance; kMarchDevice: the whole device
+// per round
+constexpr int kMarchNone = 0, kMarchGroup = 1, kMarchDevice = 2;
+MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles, int64_t most, int ninst, int nowners);
+// bytes of the march's buffers in a request for nsrc sources on grid g (the tile solver needs none)
+int64_t march_request_bytes(const eik_grid& g, int64_t nsrc, const eik_params& P);
+// Device buffers for marches of these sizes; false if they do not fit.
+bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst);
+constexpr int kMarchOverflow = 1000;  // march_run: a list was too short (see list_cap)
+MarchCtl march_ctl(const std::vector<InstDev>& inst);
+int march_run(eik_ctx* ctx, int nd, int prec, int kind, const InstDev* d_inst, int ninst, const MarchSize& sz,
+              const TTPools& pools, const void* slowpool, const MarchSeeds& sd, bool exact, bool near, FimStats* fs);
+double f32_settle();  // EIK_F32_SETTLE, EIK_MIX_SETTLE (eik_fim.hip)
+double mix_settle();
 // near: some instance has an FP64 region (unrefined mixed solve; InstDev::xlo/xhi)
 int fim_run(eik_ctx* ctx, int nd, int prec, int kind, const InstDev* d_inst, int ninst, int64_t ntiles,
             const TTPools& pools, const void* slowpool, bool exact, bool near, FimStats* fs);

@@ -126,6 +126,7 @@ extern "C" int eik_traveltime_noalloc(eik_ctx* ctx, eik_model* model, int64_t ns
     Arena A;
     A.base = slot.ptr;
     A.cap = kScratchBytes;
+    A.spare = kScratchBytes - need;
     ctx->abufs.clear();
     ctx->arena = &A;
     stats_begin(ctx);

@@ -236,6 +236,17 @@ static void worker(eik_server* S, int slot) {
                 ++it;
             }
         }
+        // what the budget leaves beside the requests goes to the march's buffers, if they fit: with
+        // less the call runs on the tile solver, so no request is held or refused for them
+        int64_t extra = 0;
+        for (int64_t k : ids) {
+            const eik_request& r = S->reqs[k].r;
+            extra += march_request_bytes(r.model->g, r.nsrc, r.params);
+        }
+        const int64_t room = S->budget_now - footprint_with(S, slot, std::max(bytes, S->held[slot]));
+        if (extra > room) extra = 0;
+        ctx->march_limit = extra;
+        bytes += extra;
         S->inflight_bytes += bytes;
         S->run[slot] = bytes;
         const Clock::time_point t0 = Clock::now();
