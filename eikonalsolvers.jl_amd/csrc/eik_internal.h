@@ -43,6 +43,7 @@ struct InstDev {
     int32_t pad2;
     const double* sinth; // 3D sphere: sin(theta_j) per theta index, computed on the host (else null)
     double band;         // band scheduler: tiles within this traveltime of the lowest pending one run
+    double mband;        // the same for the nodes a march's round may run
     double nband;        // the same for the nodes updated inside a tile
     double aband;        // adjoint rounds: tiles within this traveltime of the highest pending one run
     double rbx, rby;     // 1 / t[0], 1 / t[1]

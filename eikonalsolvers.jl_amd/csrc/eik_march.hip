@@ -416,7 +416,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
     unsigned* const pend = M.p[0] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
     const int tid = threadIdx.x, lane = tid & 63;
-    const float band = (float)I.band;
+    const float band = (float)I.mband;
     Metric<A> mcart;
 #pragma unroll
     for (int ax = 0; ax < 3; ax++) mcart.dh[ax] = (A)I.h[0];
@@ -699,7 +699,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         }
         return;
     }
-    const unsigned lim = __float_as_uint(__uint_as_float(wave_min_u32(low0)) + (float)I.band);
+    const unsigned lim = __float_as_uint(__uint_as_float(wave_min_u32(low0)) + (float)I.mband);
     Metric<A> mcart;
 #pragma unroll
     for (int ax = 0; ax < 3; ax++) mcart.dh[ax] = (A)I.h[0];
@@ -1095,7 +1095,7 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     CK(hipEventRecord(ctx->kev[0], st));
     int64_t rounds = 0;
     if (!device) {
-        constexpr int BT = 256;
+        constexpr int BT = 512;  // against 256: 600x400 x 256 21.2 -> 15.0 ms, 300x220 x 4 4.95 -> 4.67; 1024 is slower than both
         k_march_group<ND, T, SPH, MIX, NEAR, BT><<<(unsigned)ninst, BT, 0, st>>>(
             d_inst, P, M, sd.seeds, sd.cap, sd.nseed, settle, ctl, d_c);
         CK(hipGetLastError());
