@@ -47,6 +47,16 @@ constexpr unsigned kNodeBits = 27, kNodeMask = (1u << kNodeBits) - 1u;
 constexpr unsigned kHintShift = kNodeBits, kNoHint = 15u, kOnce = 0x80000000u;
 constexpr unsigned kNoEntry = 0xffffffffu;  // (no march has kNodeMask nodes)
 
+// x[i] of a uniform x, i < 2^kNodeBits.  In 3D with a 32-bit offset: one address register per access
+// rather than two, which the FP64 replay would otherwise spill (201x201x101 x 16: 63.6 -> 59.9 ms, along
+// with the view kept out of memory in hint_index).  In 2D nothing spills and the plain form is 4 % faster.
+template <int ND, typename T>
+__device__ __forceinline__ T& at(T* x, unsigned i) {
+    static_assert(sizeof(T) <= 8, "offsets of 2^27 nodes fit 32 bits");
+    if constexpr (ND == 3) return *(T*)((char*)x + i * (unsigned)sizeof(T));
+    return x[i];
+}
+
 // ------------------------------------------------------------------ one node's replay
 // A grid with its pools, per instance (wave-uniform).
 template <int ND, typename T>
@@ -158,8 +168,8 @@ __device__ __forceinline__ bool quiet_change(T v0, T k0, T v1, T k1, T settle) {
 __device__ __forceinline__ unsigned pend_bits(float p) { return max(__float_as_uint(p), 1u); }
 
 // Replays node l (on: this lane has one) and writes it if it changed; returns whether it did.
-// p: the round's pending values (only read here).  wake(k, w, q, pq, p): if w, neighbour q (the k-th
-// of 4 * ND, pending with pq) becomes pending with value p; k = 0 .. 2 * ND - 1 are the adjacent nodes.
+// p: the round's pending values (only read here).  wake(k, w, q, idle, pq, p): if w, neighbour q (the
+// k-th of 4 * ND, idle or pending with pq) becomes pending with value p; k = 0 .. 2 * ND - 1 are the adjacent nodes.
 // Nodes two away are rarely woken (only by a change of a node that they were replayed with): unless
 // some lane wakes one, wake is not called for them and *two stays false.  Every lane of the wave
 // calls it.
@@ -186,15 +196,17 @@ __device__ __forceinline__ bool relax_node(const InstDev& I, const GridView<ND, 
         ok2 |= (unsigned)in2 << k;
         q1[k] = in1 ? l + G.step(ax, g[ax], 1, k & 1) : l;
         q2[k] = in2 ? l + G.step(ax, g[ax], 2, k & 1) : l;
-        r1[k] = G.tt[q1[k]];
-        r2[k] = G.tt[q2[k]];
-        p1[k] = p[q1[k]];
+        r1[k] = at<ND>(G.tt, q1[k]);
+        r2[k] = at<ND>(G.tt, q2[k]);
+        p1[k] = at<ND>(p, q1[k]);
     }
-    const T raw = G.tt[l];
-    const T sl = G.slow[l];
+    const T raw = at<ND>(G.tt, l);
+    const T sl = at<ND>(G.slow, l);
     bool marked = signbit(raw);
+    unsigned idle1 = 0u;  // adjacent nodes that are not pending
 #pragma unroll
     for (int k = 0; k < 2 * ND; k++) {
+        idle1 |= (unsigned)(p1[k] == kIdle) << k;
         if (!((ok1 >> k) & 1u)) r1[k] = tinf<T>();
         if (!((ok2 >> k) & 1u)) r2[k] = tinf<T>();
         marked = marked || signbit(r1[k]) || signbit(r2[k]);
@@ -206,6 +218,15 @@ __device__ __forceinline__ bool relax_node(const InstDev& I, const GridView<ND, 
     } else {
         mt = mcart;
     }
+    // What the wakes need of the loads is formed here: a use of a loaded value behind the stores below
+    // would wait for those too (memory operations are counted in order).
+    float step[ND];
+#pragma unroll
+    for (int ax = 0; ax < ND; ax++) {
+        step[ax] = (float)mt.dh[ax] * (float)sl;
+        asm volatile("" : "+v"(step[ax]));
+    }
+    asm volatile("" : "+v"(idle1));
     int code[3];
     Key<T> nk;
     T nv;
@@ -270,7 +291,7 @@ __device__ __forceinline__ bool relax_node(const InstDev& I, const GridView<ND, 
     const bool kchg = nv < tinf<T>() && !keq(nk, k0);
     const bool chg = on && (vchg || kchg);
     if (chg) {
-        G.tt[l] = nk.D ? -nv : nv;
+        at<ND>(G.tt, l) = nk.D ? -nv : nv;
         if (nk.D != k0.D) G.dd[lin] = (uint8_t)nk.D;
         if (nk.D) {
             G.kk[lin] = nk.K;
@@ -282,29 +303,40 @@ __device__ __forceinline__ bool relax_node(const InstDev& I, const GridView<ND, 
     const T ck = k0.K < nk.K ? k0.K : nk.K;
     const T c = reach_key(ck);
     const float cf = (float)ck;
+    // adjacent nodes whose key the change reaches; of the nodes two away, which use this one only
+    // through the node between, those whose key it reaches and whose node between pops no later (an
+    // unreached one is pending already: the node between was reached)
     unsigned w1 = 0u, w2 = 0u;
 #pragma unroll
     for (int k = 0; k < 2 * ND; k++) {
-        const bool i1 = (ok1 >> k) & 1u, i2 = (ok2 >> k) & 1u;
-        const bool x1 = (f1 >> k) & 1u, x2 = (f2 >> k) & 1u, k1m = (m1 >> k) & 1u, k2m = (m2 >> k) & 1u;
-        const bool a = loud && i1 && !x1 && (k1m || v1[k] >= c);
-        // a node two away uses this one only through the node between, and only if that one pops
-        // no later than it does (an unreached one is pending already: the node between was reached)
-        const bool b = loud && i2 && !x2 && v2[k] < tinf<T>() && v1[k] < tinf<T>() &&
-                       (k2m || (v2[k] >= c && (k1m || reach_key(v1[k]) <= v2[k])));
-        w1 |= (unsigned)a << k;
-        w2 |= (unsigned)b << k;
+        const bool r = (v2[k] < tinf<T>()) & (v1[k] < tinf<T>());
+        const bool far = (v2[k] >= c) & (reach_key(v1[k]) <= v2[k]);
+        w1 |= (unsigned)(v1[k] >= c) << k;
+        w2 |= (unsigned)(r & far) << k;
     }
+    if (!fast) {  // a marked node's key is not its value: woken whatever it is, unless an init node
+#pragma unroll
+        for (int k = 0; k < 2 * ND; k++) {
+            const bool r = (v2[k] < tinf<T>()) & (v1[k] < tinf<T>());
+            const bool k1m = (m1 >> k) & 1u, k2m = (m2 >> k) & 1u;
+            w1 |= (unsigned)k1m << k;
+            w2 |= (unsigned)(r & (k2m | ((v2[k] >= c) & k1m))) << k;
+        }
+        w1 &= ~f1;
+        w2 &= ~f2;
+    }
+    w1 = loud ? w1 & ok1 : 0u;
+    w2 = loud ? w2 & ok2 : 0u;
 #pragma unroll
     for (int k = 0; k < 2 * ND; k++)
-        wake(k, (w1 >> k) & 1u, q1[k], p1[k], fmaxf(cf, fminf((float)v1[k], cf + (float)mt.dh[k >> 1] * (float)sl)));
+        wake(k, (w1 >> k) & 1u, q1[k], (idle1 >> k) & 1u, p1[k], fmaxf(cf, fminf((float)v1[k], cf + step[k >> 1])));
     *two = __ballot(w2 != 0u) != 0ull;
     if (*two) {
         unsigned p2[2 * ND];
 #pragma unroll
-        for (int k = 0; k < 2 * ND; k++) p2[k] = p[((w2 >> k) & 1u) ? q2[k] : l];
+        for (int k = 0; k < 2 * ND; k++) p2[k] = at<ND>(p, ((w2 >> k) & 1u) ? q2[k] : l);
 #pragma unroll
-        for (int k = 0; k < 2 * ND; k++) wake(2 * ND + k, (w2 >> k) & 1u, q2[k], p2[k], fmaxf(cf, (float)v2[k]));
+        for (int k = 0; k < 2 * ND; k++) wake(2 * ND + k, (w2 >> k) & 1u, q2[k], p2[k] == kIdle, p2[k], fmaxf(cf, (float)v2[k]));
     }
     return chg;
 }
@@ -321,7 +353,7 @@ __device__ __forceinline__ bool may_run(const GridView<ND, T>& G, const unsigned
     for (int k = 0; k < 4 * ND; k++) {
         const int ax = k >> 2, d = (k & 2) ? 2 : 1;
         const bool in = (k & 1) ? g[ax] >= d : g[ax] + d < G.n[ax];
-        v[k] = p[in ? l + G.step(ax, g[ax], d, k & 1) : l];
+        v[k] = at<ND>(p, in ? l + G.step(ax, g[ax], d, k & 1) : l);
         // outside the grid nothing holds it up; a node further down also wins a tie
         v[k] = in ? v[k] - (unsigned)(k & 1) : kIdle;
     }
@@ -344,7 +376,8 @@ __device__ __forceinline__ unsigned hint_index(const GridView<ND, T>& G, unsigne
     constexpr unsigned S = GridView<ND, T>::E == 8 ? 3u : 2u;
     const int c = (int)((l >> (S * (unsigned)ax)) & (unsigned)(GridView<ND, T>::E - 1));
     const unsigned s = 1u << (S * (unsigned)ax);
-    const unsigned b = ax == 0 ? G.bs[0] : (ax == 1 ? G.bs[1] : G.bs[2]);
+    // (not a choice between the three: the compiler would put the view in memory and choose an address)
+    const unsigned b = (G.bs[0] & (0u - (ax == 0))) | (G.bs[1] & (0u - (ax == 1))) | (G.bs[2] & (0u - (ax == 2)));
     const unsigned in = (unsigned)d * s, out = b - (unsigned)(GridView<ND, T>::E - d) * s;
     if (k & 1u) return l - (c >= d ? in : out);
     return l + (c + d < GridView<ND, T>::E ? in : out);
@@ -427,7 +460,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
     };
     auto get = [&](int k, unsigned at) { return at < (unsigned)kGroupList ? s_list[k][at] : sp[(size_t)k * lcap + (at - kGroupList)]; };
     auto lower = [&](unsigned q, unsigned p) {
-        (void)__hip_atomic_fetch_min(&pend[q], p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        (void)__hip_atomic_fetch_min(&at<ND>(pend, q), p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     if (tid < 3) {
         s_cnt[tid] = 0u;
@@ -466,10 +499,10 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
             if (have) {
                 const unsigned e = get(cur, i);
                 l = e & kNodeMask;
-                const unsigned at = own[l];
-                p = pend[l];
+                const unsigned ow = at<ND>(own, l);
+                p = at<ND>(pend, l);
                 run = may_run<ND, T>(G, pend, l, p, &hold) && p <= lim;
-                have = (e & kOnce) || at == i;
+                have = (e & kOnce) || ow == i;
                 run = run && have;
             }
             const unsigned long long mr = __ballot(run);
@@ -505,38 +538,37 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
             const unsigned j = b + lane;
             const bool on = j < nrun;
             const unsigned l = s_run[on ? j : b];
-            if (on) pend[l] = kIdle;
             unsigned who[4 * ND] = {}, fresh = 0u;
             bool two;
             const bool chg = relax_node<ND, T, SPH, MIX, NEAR>(
-                I, G, mcart, pend, l, on, stl, &two, [&](int k, bool w, unsigned q, unsigned pq, float p) {
+                I, G, mcart, pend, l, on, stl, &two, [&](int k, bool w, unsigned q, bool idle, unsigned, float p) {
                     who[k] = q;
                     if (w) {
                         const unsigned pu = pend_bits(p);
                         lowest = min(lowest, pu);
                         lower(q, pu);
                     }
-                    fresh |= (unsigned)(w && pq == kIdle) << k;
+                    fresh |= (unsigned)(w & idle) << k;
                 });
-            unsigned off[4 * ND], total = 0u;
+            if (on) at<ND>(pend, l) = kIdle;  // (no node of the round wakes it)
+            unsigned total = 0u;
 #pragma unroll
-            for (int k = 0; k < 4 * ND; k++) {
-                off[k] = 0u;
-                if (k < 2 * ND || two) {
-                    const unsigned long long m = __ballot((fresh >> k) & 1u);
-                    off[k] = total + lane_rank(m);
-                    total += (unsigned)__popcll(m);
-                }
-            }
+            for (int k = 0; k < 4 * ND; k++)
+                if (k < 2 * ND || two) total += (unsigned)__popcll(__ballot((fresh >> k) & 1u));
             if (total) {
                 unsigned base = 0u;
                 if (lane == 0) base = atomicAdd(&s_cnt[nslot], total);
                 base = (unsigned)__builtin_amdgcn_readfirstlane((int)base);
 #pragma unroll
                 for (int k = 0; k < 4 * ND; k++) {
-                    if ((k < 2 * ND || two) && ((fresh >> k) & 1u)) {
-                        put(cur ^ 1, base + off[k], who[k]);
-                        own[who[k]] = base + off[k];
+                    if (k < 2 * ND || two) {
+                        const unsigned long long m = __ballot((fresh >> k) & 1u);
+                        const unsigned to = base + lane_rank(m);
+                        if ((fresh >> k) & 1u) {
+                            put(cur ^ 1, to, who[k]);
+                            at<ND>(own, who[k]) = to;
+                        }
+                        base += (unsigned)__popcll(m);
                     }
                 }
             }
@@ -681,7 +713,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
     const unsigned lo = min(cnt, blk * part), hi = min(cnt, lo + part);
     // the nodes this block ran in the last round become idle in the buffer of that round
     const auto clear_ran = [&] {
-        for (unsigned i = tid; i < nran; i += kRoundThreads) pr[ran[1 + i]] = kIdle;
+        for (unsigned i = tid; i < nran; i += kRoundThreads) at<ND>(pr, ran[1 + i]) = kIdle;
     };
     if (lo >= hi) {
         clear_ran();
@@ -716,7 +748,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             s_nfresh = 0u;
         }
         lds_barrier();  // also: every thread has read the run list of the last round
-        unsigned e[kRoundPer], pv[kRoundPer], pb[kRoundPer], at[kRoundPer];
+        unsigned e[kRoundPer], pv[kRoundPer], pb[kRoundPer], pos[kRoundPer];
 #pragma unroll
         for (int u = 0; u < kRoundPer; u++) {
             // entry i lies in the segment whose end is the first beyond i
@@ -724,8 +756,8 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             unsigned s = (unsigned)__popcll(__ballot(end <= i0));
             if (i < hi)
                 while (s_end[wave][s] <= i) s++;
-            at[u] = s * scap + (i - (s ? s_end[wave][s - 1] : 0u));
-            e[u] = i < hi ? from[at[u]] : kNoEntry;
+            pos[u] = s * scap + (i - (s ? s_end[wave][s - 1] : 0u));
+            e[u] = i < hi ? from[pos[u]] : kNoEntry;
         }
         if (base == lo) clear_ran();
         // own value, that of the node that held it up before, and a lowered one, in one round trip
@@ -734,10 +766,10 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         for (int u = 0; u < kRoundPer; u++) {
             const bool have = e[u] != kNoEntry;
             const unsigned l = have ? e[u] & kNodeMask : 0u, h = (e[u] >> kHintShift) & 15u;
-            pv[u] = p[l];
-            pb[u] = p[hints && have && h != kNoHint ? hint_index<ND, T>(G, l, h) : l];
-            ow[u] = own[have && !(e[u] & kOnce) ? l : 0u];
-            ls[u] = less[l];
+            pv[u] = at<ND>(p, l);
+            pb[u] = at<ND>(p, hints && have && h != kNoHint ? hint_index<ND, T>(G, l, h) : l);
+            ow[u] = at<ND>(own, have && !(e[u] & kOnce) ? l : 0u);
+            ls[u] = at<ND>(less, l);
         }
         // the other stencil positions of the entries that are not held up still, in another
         unsigned hold[kRoundPer];
@@ -745,7 +777,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
 #pragma unroll
         for (int u = 0; u < kRoundPer; u++) {
             const unsigned h = (e[u] >> kHintShift) & 15u;
-            if (e[u] != kNoEntry && !(e[u] & kOnce) && ow[u] != at[u]) e[u] = kNoEntry;
+            if (e[u] != kNoEntry && !(e[u] & kOnce) && ow[u] != pos[u]) e[u] = kNoEntry;
             // still held up: lower, or as low and further down
             const bool held = hints && h != kNoHint && (pb[u] < pv[u] || ((h & 1u) && pb[u] == pv[u]));
             run[u] = e[u] != kNoEntry && pv[u] <= lim && !held;
@@ -782,7 +814,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
                 if (keep) {
                     const unsigned pk = min(pv[u], ls[u]);
                     s_keep[b] = l | hold[u] << kHintShift | kOnce;
-                    pn[l] = pk;
+                    at<ND>(pn, l) = pk;
                     lowest = min(lowest, pk);
                 }
             }
@@ -794,42 +826,38 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             const bool on = j < nrun;
             const unsigned l = s_run[on ? j : b];
             if (on) {
-                pn[l] = kIdle;
-                pr[l] = kIdle;
-                less[l] = kIdle;
+                at<ND>(pn, l) = kIdle;
+                at<ND>(pr, l) = kIdle;
+                at<ND>(less, l) = kIdle;
                 ran[1 + j] = l;
             }
             unsigned who[4 * ND] = {}, fresh = 0u;
             bool two;
             const bool chg = relax_node<ND, T, SPH, MIX, NEAR>(
-                I, G, mcart, p, l, on, settle, &two, [&](int k, bool w, unsigned q, unsigned pq, float pf) {
+                I, G, mcart, p, l, on, settle, &two, [&](int k, bool w, unsigned q, bool idle, unsigned pq, float pf) {
                     who[k] = q;
                     const unsigned pu = pend_bits(pf);
                     if (w && pu < pq) {
                         lowest = min(lowest, pu);
-                        atomicMin(pq == kIdle ? &pn[q] : &less[q], pu);
+                        atomicMin(idle ? &at<ND>(pn, q) : &at<ND>(less, q), pu);
                     }
-                    fresh |= (unsigned)(w && pq == kIdle) << k;
+                    fresh |= (unsigned)(w & idle) << k;
                 });
-            unsigned off[4 * ND], total = 0u;
+            unsigned total = 0u;
 #pragma unroll
-            for (int k = 0; k < 4 * ND; k++) {
-                off[k] = 0u;
-                if (k < 2 * ND || two) {
-                    const unsigned long long m = __ballot((fresh >> k) & 1u);
-                    off[k] = total + lane_rank(m);
-                    total += (unsigned)__popcll(m);
-                }
-            }
+            for (int k = 0; k < 4 * ND; k++)
+                if (k < 2 * ND || two) total += (unsigned)__popcll(__ballot((fresh >> k) & 1u));
             if (total) {
                 unsigned to_at = 0u;
                 if (lane == 0) to_at = atomicAdd(&s_nfresh, total);
                 to_at = (unsigned)__builtin_amdgcn_readfirstlane((int)to_at);
 #pragma unroll
                 for (int k = 0; k < 4 * ND; k++) {
-                    if ((k < 2 * ND || two) && ((fresh >> k) & 1u)) {
-                        const unsigned f = to_at + off[k];
-                        if (f < (unsigned)kRoundFresh) s_fresh[f] = who[k];
+                    if (k < 2 * ND || two) {
+                        const unsigned long long m = __ballot((fresh >> k) & 1u);
+                        const unsigned f = to_at + lane_rank(m);
+                        if (((fresh >> k) & 1u) && f < (unsigned)kRoundFresh) s_fresh[f] = who[k];
+                        to_at += (unsigned)__popcll(m);
                     }
                 }
             }
@@ -842,9 +870,9 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         for (unsigned i = tid; i < nkeep; i += kRoundThreads)
             if (out + i < scap) to[out + i] = s_keep[i];
         for (unsigned i = tid; i < min(nfresh, (unsigned)kRoundFresh); i += kRoundThreads) {
-            const unsigned at = out + nkeep + i;
-            if (at < scap) to[at] = s_fresh[i] | kNoHint << kHintShift;
-            own[s_fresh[i]] = blk * scap + at;
+            const unsigned j = out + nkeep + i;
+            if (j < scap) to[j] = s_fresh[i] | kNoHint << kHintShift;
+            at<ND>(own, s_fresh[i]) = blk * scap + j;
         }
         out = min(out + nkeep + min(nfresh, (unsigned)kRoundFresh), scap);
     }
