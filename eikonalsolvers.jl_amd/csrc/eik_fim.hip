@@ -868,7 +868,9 @@ __global__ void k_fine_setup(const FineDev* __restrict__ fine, int nfine, const 
 // solution and its pop keys: k_c = min key over coarse-coincident nodes, k_stop = min key over
 // face nodes with key >= k_c, transfer = coarse-coincident nodes with key <= k_stop.  One block
 // per source; the transferred points are listed in coarse-window order (xlist, cap entries per
-// source) and k_stop is stored in the fine instance for the adjoint.
+// source) and k_stop is stored in the fine instance for the adjoint.  A block looks at the coincident
+// and the face nodes alone and lists its chunks by prefix sums (one thread listing them after two passes over
+// the whole box: 0.55 ms at 31^3 nodes, 41 us so).
 template <typename T>
 __global__ void __launch_bounds__(256) k_transfer(const FineDev* __restrict__ fine, InstDev* __restrict__ finst,
                                                   TTPools fp, const InstDev* __restrict__ cinst, T* __restrict__ ttc,
@@ -879,21 +881,21 @@ __global__ void __launch_bounds__(256) k_transfer(const FineDev* __restrict__ fi
     const FineDev F = fine[f];
     const InstDev I = finst[f];
     const InstDev C = cinst[F.cinst];
-    const int64_t n = (int64_t)I.n[0] * I.n[1] * I.n[2];
     const double* ttf = (const double*)fp.tt + I.tt_off;
     const double* kf = (const double*)fp.k + I.tt_off;
     const double* sf = (const double*)fp.s + I.tt_off;
     const uint8_t* df = fp.d + I.tt_off;
     __shared__ Key<double> red[256];
-    auto coord = [&](int64_t l, int* g) {
-        g[0] = (int)(l % I.n[0]);
-        g[1] = (int)((l / I.n[0]) % I.n[1]);
-        g[2] = (int)(l / ((int64_t)I.n[0] * I.n[1]));
-    };
-    auto coincident = [&](const int* g) {
-        for (int d = 0; d < nd; d++)
-            if (g[d] % F.df != 0) return false;
-        return true;
+    __shared__ int s_cnt[4];
+    int nw[3] = {1, 1, 1};  // coarse-coincident nodes along each axis
+    for (int d = 0; d < nd; d++) nw[d] = (I.n[d] - 1) / F.df + 1;
+    const int nwin = nw[0] * nw[1] * nw[2];
+    // the w-th of them, x fastest
+    auto window = [&](int w, int* c) {
+        c[0] = w % nw[0];
+        c[1] = (w / nw[0]) % nw[1];
+        c[2] = w / (nw[0] * nw[1]);
+        return (int64_t)c[0] * F.df + (int64_t)I.n[0] * ((int64_t)c[1] * F.df + (int64_t)I.n[1] * ((int64_t)c[2] * F.df));
     };
     // pop key of a fine node; init nodes pop before every other node
     auto keyof = [&](int64_t l) {
@@ -915,54 +917,61 @@ __global__ void __launch_bounds__(256) k_transfer(const FineDev* __restrict__ fi
     };
     const Key<double> kinf{EIK_INF, EIK_INF, 0};
     Key<double> m = kinf;
-    for (int64_t l = threadIdx.x; l < n; l += 256) {
-        int g[3];
-        coord(l, g);
-        if (coincident(g)) {
-            const Key<double> k = keyof(l);
-            if (klt(k, m)) m = k;
-        }
+    for (int w = threadIdx.x; w < nwin; w += 256) {
+        int c[3];
+        const Key<double> k = keyof(window(w, c));
+        if (klt(k, m)) m = k;
     }
     const Key<double> kc = blockmin(m);
     m = kinf;
-    for (int64_t l = threadIdx.x; l < n; l += 256) {
-        int g[3];
-        coord(l, g);
-        if (signbit(ttf[l]) || !(ttf[l] < EIK_INF)) continue;  // init nodes are never popped
-        bool face = false;
-        for (int d = 0; d < nd; d++) {
-            if (g[d] == 0 && !F.outmin[d]) face = true;
-            if (g[d] == I.n[d] - 1 && !F.outmax[d]) face = true;
+    for (int side = 0; side < 2 * nd; side++) {  // the faces that are not model borders
+        const int d = side >> 1;
+        if (side & 1 ? F.outmax[d] : F.outmin[d]) continue;
+        const int a = d == 0 ? 1 : 0, b = d == 2 ? 1 : 2;
+        const int64_t st[3] = {1, I.n[0], (int64_t)I.n[0] * I.n[1]};
+        const int64_t at = (side & 1 ? I.n[d] - 1 : 0) * st[d];
+        for (int i = threadIdx.x; i < I.n[a] * I.n[b]; i += 256) {
+            const int64_t l = at + (i % I.n[a]) * st[a] + (i / I.n[a]) * st[b];
+            if (signbit(ttf[l]) || !(ttf[l] < EIK_INF)) continue;  // init nodes are never popped
+            const Key<double> k = keyof(l);
+            if (!klt(k, kc) && klt(k, m)) m = k;
         }
-        const Key<double> k = keyof(l);
-        if (face && !klt(k, kc) && klt(k, m)) m = k;
     }
     const Key<double> ks = blockmin(m);
-    if (threadIdx.x != 0) return;
-    finst[f].tstopK = ks.K;
-    finst[f].tstopS = ks.S;
-    finst[f].tstopD = ks.D;
-    int nw[3] = {1, 1, 1};
-    for (int d = 0; d < nd; d++) nw[d] = (I.n[d] - 1) / F.df + 1;
+    if (threadIdx.x == 0) {
+        finst[f].tstopK = ks.K;
+        finst[f].tstopS = ks.S;
+        finst[f].tstopD = ks.D;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int cnt = 0;
-    for (int wz = 0; wz < nw[2]; wz++)
-        for (int wy = 0; wy < nw[1]; wy++)
-            for (int wx = 0; wx < nw[0]; wx++) {
-                const int64_t lf = (int64_t)wx * F.df +
-                                   (int64_t)I.n[0] * ((int64_t)wy * F.df + (int64_t)I.n[1] * ((int64_t)wz * F.df));
-                if (!(fabs(ttf[lf]) < EIK_INF) || klt(ks, keyof(lf))) continue;
-                const double t = fabs(ttf[lf]);
-                const int cg[3] = {F.i1c[0] + wx, F.i1c[1] + wy, F.i1c[2] + wz};
-                const int64_t lc = cg[0] + (int64_t)C.n[0] * (cg[1] + (int64_t)C.n[1] * cg[2]);
-                ttc[C.tt_off + lc] = -(T)t;
-                if (dpool)
-                    dpool[C.tt_off + lc] = (uint8_t)kInitDepth;
-                else
-                    seed_tiles_fwd(C, nd, cg, cflags, cpend, t);
-                if (cnt < cap) xlist[(int64_t)f * cap + cnt] = SrcPt{F.cinst, (int32_t)lf, lc};
-                cnt++;
-            }
-    ntransfer[f] = cnt;
+    for (int base = 0; base < nwin; base += 256) {
+        const int w = base + threadIdx.x;
+        int c[3] = {0, 0, 0};
+        const int64_t lf = w < nwin ? window(w, c) : 0;
+        const double t = fabs(ttf[lf]);
+        const bool on = w < nwin && t < EIK_INF && !klt(ks, keyof(lf));
+        const unsigned long long mask = __ballot(on);
+        if (lane == 0) s_cnt[wave] = __popcll(mask);
+        __syncthreads();
+        int at = cnt + __popcll(mask & ((1ull << lane) - 1ull));
+        for (int v = 0; v < 4; v++) {
+            at += v < wave ? s_cnt[v] : 0;
+            cnt += s_cnt[v];
+        }
+        if (on) {
+            const int cg[3] = {F.i1c[0] + c[0], F.i1c[1] + c[1], F.i1c[2] + c[2]};
+            const int64_t lc = cg[0] + (int64_t)C.n[0] * (cg[1] + (int64_t)C.n[1] * cg[2]);
+            ttc[C.tt_off + lc] = -(T)t;
+            if (dpool)
+                dpool[C.tt_off + lc] = (uint8_t)kInitDepth;
+            else
+                seed_tiles_fwd(C, nd, cg, cflags, cpend, t);
+            if (at < cap) xlist[(int64_t)f * cap + at] = SrcPt{F.cinst, (int32_t)lf, lc};
+        }
+        __syncthreads();  // the next chunk's counts
+    }
+    if (threadIdx.x == 0) ntransfer[f] = cnt;
 }
 
 // receiver picks: bilinear_interp (eikforward2D.jl:17-87) / trilinear_interp (eikforward3D.jl:17-140)
