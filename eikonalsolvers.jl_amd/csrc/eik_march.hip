@@ -1095,7 +1095,7 @@ static T tinf_host() {
     return (T)INFINITY;
 }
 
-constexpr int kMarchBatch = 8;  // rounds enqueued between two looks at what is left
+constexpr int kMarchBatch = 32;  // rounds enqueued between two looks at what is left
 
 template <int ND, typename T, bool SPH, bool MIX, bool NEAR>
 static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const MarchSize& sz, const TTPools& P, const T* slowpool,
