@@ -984,19 +984,22 @@ static void march_bytes(int64_t ntiles, int64_t stiles, int64_t most, int ninst,
 
 // Which solver runs an instance set (EIK_MARCH overrides: kMarch*).  A workgroup per instance costs
 // about the same for one instance as for one per CU, and grows with the instance's nodes; the
-// whole-device rounds cost about 13 us each whatever they hold, until the device is full; the tile
-// solver needs fewer, longer rounds, which wins on few large 2D grids.  Milliseconds per call, FP64,
-// tiles / workgroup / device:
-//   2D   300x240 x 1   6.5 /  4.4 /  8.8    600x480 x 64   37.8 / 19.0 / 35.6
-//        1200x960 x 1  37.7 / 52.2 / 49.3   1200x960 x 4   53.3 / 52.3 / 50.9   1200x960 x 16  93.4 / 58.2 / 76.2
-//   3D   24^3 x 4      4.5 /  3.6 /  3.1    24^3 x 16       6.7 /  3.7 /  4.0
-//        48x48x28 x 16 10.3 / 6.1 /  5.3    48x48x28 x 64  16.4 /  6.5 /  7.5   64x64x38 x 64   23.5 / 11.9 / 11.2
-//        100x100x60 x 1 12.0 / 33 / 8.1     200x200x120 x 4 75.2 / 772 / 38.3
-// Mixed sweeps are cheaper in the tile solver (600x480 x 1: 9.4 / 12.3, x 16: 17.8 / 14.2; 1200x960 x 16:
-// 49.8 / 61.0; 3D as FP64: 200x200x120 x 4 54.6 / - / 36.5), and so are FP32 ones: it wins beyond 300x240 (x 1:
-// 4.6 / 4.8) and 100x100x60 (x 64: 30.6 / - / 27.2; 150x150x90 x 16: 33.6 / - / 33.4; 200x200x120 x 1: 21.7 / - / 25.7).
-// FP32 spheres stay with it: within FP32 resolution their many near-ties have several fixed points, and
-// the march can circulate among them until it settles (600x600 x 8: 31 ms, the march 579).
+// whole-device rounds cost about 12 us each whatever they hold, until the device is full; the tile
+// solver needs fewer, longer rounds, which wins where its sweeps are cheap and instances few and large.
+// Milliseconds per call, tiles / workgroup / device:
+//   2D FP64   300x240 x 1   6.5 /  4.1 /  8.5    600x480 x 64   37.5 / 11.3 / 22.0
+//             1200x960 x 1  37.8 / 36.5 / 34.5   1200x960 x 4   52.8 / 38.7 / 34.1   1200x960 x 16 93.4 / 44.1 / 42.9
+//             2400x1920 x 4 175 / 206 / 98       600x600 sphere x 8 50.8 / 28.2 / 31.2 (mixed the same)
+//   2D mixed  600x480 x 1   9.3 /  8.9 / 14.5    1200x960 x 4   29.4 / 38.2 / 33.3   1200x960 x 16 48.5 / 43.9 / 42.1
+//   2D FP32   300x240 x 1   4.5 /  3.6 /  8.4    600x480 x 4     9.3 /  9.4 / 16.0   600x480 x 16  14.5 /  9.8 / 15.6
+//             1200x960 x 16 36.9 / 42.8 / 43.8
+//   3D FP64   24^3 x 4      4.0 /  2.7 /  2.6    24^3 x 16       6.1 /  2.9 /  3.3   24^3 sphere x 1 1.5 / 1.2 / 1.7
+//             48x48x28 x 16 9.7 /  5.4 /  4.6    48x48x28 x 64  15.7 /  6.2 /  6.8   64x64x38 x 64  23.3 / 11.9 / 10.8
+//             100x100x60 x 1 11.3 / 32 / 6.7     200x200x120 x 4 74.6 / 1032 / 29.6 (mixed 54.2 / - / 28.9)
+//   3D FP32   48x48x28 x 1  3.5 /  4.5 /  3.9    150x150x90 x 1 15.0 / - / 12.2      150x150x90 x 16 33.0 / - / 26.2
+//             200x200x120 x 1 20.9 / - / 20.6    200x200x120 x 4 29.2 / - / 25.8     201x201x101 x 16 48.9 / - / 44.4
+// FP32 spheres stay with the tiles: within FP32 resolution their many near-ties have several fixed points,
+// and the march can circulate among them until it settles (600x600 x 8: 31 ms, the march 579).
 MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles, int64_t most, int ninst, int nowners) {
     const bool f32 = prec == EIK_PREC_FP32, sph = kind == EIK_GRID2D_SPHERE || kind == EIK_GRID3D_SPHERE;
     MarchSize z{ntiles, stiles, most, f32 ? sizeof(float) : sizeof(double), nullptr, nowners, kMarchNone};
@@ -1005,13 +1008,17 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
         return z;
     }
     const int64_t nodes = most * 64;
-    if (f32 && (sph || nodes > (nd == 2 ? 80000 : 700000))) return z;
-    if (nd == 2 && prec == EIK_PREC_MIXED)
-        z.mode = nodes <= 160000 || (nodes <= 400000 && ninst >= 16) ? kMarchGroup : kMarchNone;
+    if (f32 && sph) return z;
+    if (nd == 2 && f32)
+        z.mode = nodes <= 150000 || (nodes <= 400000 && ninst >= 8) ? kMarchGroup : kMarchNone;
+    else if (nd == 2 && prec == EIK_PREC_MIXED && !sph)
+        z.mode = nodes <= 320000 || (nodes <= 1200000 && ninst >= 16) ? kMarchGroup : kMarchNone;
     else if (nd == 2)
-        z.mode = nodes <= 400000 || ninst >= 8 ? kMarchGroup : (ninst >= 4 ? kMarchDevice : kMarchNone);
+        z.mode = nodes <= 800000 || ninst >= 32 ? kMarchGroup : kMarchDevice;
+    else if (f32 && nodes > (ninst >= 4 ? 6000000 : 3000000))
+        z.mode = kMarchNone;
     else
-        z.mode = nodes <= 1500 * (int64_t)ninst ? kMarchGroup : kMarchDevice;
+        z.mode = nodes <= std::max<int64_t>(16000, 1500 * (int64_t)ninst) ? kMarchGroup : kMarchDevice;
     return z;
 }
 
