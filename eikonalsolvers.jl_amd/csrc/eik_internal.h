@@ -402,6 +402,7 @@ struct eik_ctx {
     bool split = true;         // large calls may split their sources with the peer
     bool in_split = false;     // the current call is split (set on the context and its peer)
     int64_t march_limit = -1;  // bytes the march's buffers may grow by in this call (-1: no limit)
+    bool shared_device = false;  // other calls keep the device busy beside this one (see forward_solve)
     bool tiles_only = false;   // the tile solver instead of a march (see forward_solve)
     int xcap = 1;  // capacity per source of the transferred-point list
     std::mutex mu;
