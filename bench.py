@@ -28,12 +28,12 @@ import numpy as np  # noqa: E402
 
 METRIC = "source-solves/s + gradient evals/s, 3D 201²×101 grid; serving p50/p99 latency"
 HBM_PEAK_GBS = 8000.0
-TILE_NODES_3D = 64  # forward tiles are 4x4x4 (one wavefront each)
-# algorithmic bytes per node-visit: slowness + traveltime read + traveltime write (FP64 pools for
+TILE_NODES_3D = 64  # tile_activations counts 64 node replays (the tile solver's unit, one wavefront)
+# algorithmic bytes per replay: slowness + traveltime read + traveltime write (FP64 pools for
 # fp64 and mixed, FP32 pools for fp32)
 BYTES_PER_VISIT = {"fp64": 24, "mixed": 24, "fp32": 12}
-KERNELS = {"fp64": "k_fim_round<3,double,false,false,false>", "mixed": "k_fim_round<3,double,false,true,false>",
-           "fp32": "k_fim_round<3,float,false,false,false>"}
+KERNELS = {"fp64": "k_march_round<3,double,false,false,false>", "mixed": "k_march_round<3,double,false,true,false>",
+           "fp32": "k_march_round<3,float,false,false,false>"}
 
 
 def run_steps(model, src, recs, ep, steps, warmup):
@@ -114,8 +114,8 @@ def serving_leg(n_req: int, nslots: int) -> dict:
 def _traffic_from_profile(prec: str):
     """HBM bytes per round-kernel launch of one precision, measured with rocprofv3 FETCH_SIZE /
     WRITE_SIZE (scaled by the same counters on a plain copy) and committed under profiles/ as
-    k_fim_round_3d_<prec>_traffic.json; None if absent."""
-    p = os.path.join(ROOT, "profiles", f"k_fim_round_3d_{prec}_traffic.json")
+    k_march_round_3d_<prec>_traffic.json; None if absent."""
+    p = os.path.join(ROOT, "profiles", f"k_march_round_3d_{prec}_traffic.json")
     if not os.path.exists(p):
         return None
     with open(p) as f:
@@ -136,10 +136,10 @@ def _roofline(prec: str, f: dict) -> dict:
         "traffic": None,
         "traffic_scope": "HBM bytes per launch of this kernel (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a plain "
                          "copy of known size)",
-        "achieved_scope": "algorithmic bytes per launch / average launch duration (HIP events on the stream each "
-                          "launch runs on); the call's sources are split over two streams whose launches overlap, "
-                          "so achieved_device = algorithmic bytes of the step's launches / time in which at least "
-                          "one of them ran",
+        "achieved_scope": "algorithmic bytes per round launch of the coarse grids' marches / average duration of a "
+                          "round, gaps included (HIP events around each march, on its stream); the call's sources "
+                          "are split over two streams whose marches overlap, so achieved_device = algorithmic bytes "
+                          "of the step / time in which at least one of them ran",
         "achieved_device": round(f["achieved_gbs"], 2) if f["achieved_gbs"] else None,
         "frac_device": round(f["achieved_gbs"] / HBM_PEAK_GBS, 5) if f["achieved_gbs"] else None,
         "kernel_busy_ms_per_step": round(f["kernel_busy_ms_per_step"], 3),
@@ -147,7 +147,7 @@ def _roofline(prec: str, f: dict) -> dict:
         "algorithmic_bytes_per_launch": round(alg_per_launch),
         "launches_per_step": launches,
         "avg_launch_us": round(1e3 * f["kernel_all_ms_per_step"] / max(launches, 1.0), 2),
-        "launch_scope": "every launch of this instantiation in a step (FP64: the refined boxes' solve too)",
+        "launch_scope": "rounds of the coarse grids' marches, one launch each, to within a batch of 32",
         "node_visits_per_step": f["node_visits_per_step"],
         "visits_per_node": round(f["visits_per_node"], 3),
         "updates_per_node": round(f["updates_per_node"], 3),
@@ -159,8 +159,8 @@ def _roofline(prec: str, f: dict) -> dict:
     tr = _traffic_from_profile(prec)
     if tr is not None:
         out["traffic"] = tr["hbm_bytes_per_launch"]
-        out["traffic_bytes_per_step"] = round(tr["hbm_bytes_per_launch"] * launches)
-        out["traffic_over_algorithmic"] = round(tr["hbm_bytes_per_launch"] / max(alg_per_launch, 1.0), 3)
+        out["traffic_bytes_per_step"] = round(tr["hbm_bytes_per_launch"] * tr["launches"])
+        out["traffic_over_algorithmic"] = round(out["traffic_bytes_per_step"] / max(alg_per_launch * launches, 1.0), 3)
         out["traffic_measured_on"] = tr.get("measured_on", "")
     return out
 
@@ -272,14 +272,8 @@ def main() -> int:
         kern_ms = tot["_kernel_ms"]
         visits = tot["tile_activations"] * TILE_NODES_3D
         nn = args.steps * nsrc * grd.npts
-        # the round kernel as a profiler sees it: in FP64 the refined boxes around the sources are
-        # solved by the same kernel instantiation as the coarse grid, so their launches count too
-        k_ms, k_visits, k_launches, k_busy = kern_ms, visits, tot["launches"], tot["kernel_busy_ms"]
-        if prec == "fp64":
-            k_ms += tot["fine_kernel_ms"]
-            k_visits += tot["fine_tile_activations"] * TILE_NODES_3D
-            k_launches += tot["fine_launches"]
-            k_busy = tot["all_kernel_busy_ms"]
+        # a march is one span of back-to-back round launches
+        k_ms, k_visits, k_launches, k_busy = kern_ms, visits, tot["rounds"], tot["kernel_busy_ms"]
         res[prec] = {
             "solves_per_s": nsrc * args.steps / dt,
             "ms_per_step": 1e3 * dt / args.steps,
