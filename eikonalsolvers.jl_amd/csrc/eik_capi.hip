@@ -207,7 +207,10 @@ const char* eik_last_error(const eik_ctx* ctx) { return ctx ? ctx->err.c_str() :
 // source-nodes stay on one stream: there the halves' rounds are too small to fill the device and
 // the split costs time (1-2 x 2^22 source-nodes: 600x400 x 18 and x 32 sources 20-23 % slower,
 // 161x161x81 x 4 10 %, 101x101x51 x 9 14 %; 300x220 x 4: 6 %), from about 3.7 x 2^22 it gains
-// (600x400 x 64 +4 %, 161x161x81 x 8 +4 %, the larger workloads above).  Results do not depend on
+// (600x400 x 64 +4 %, 161x161x81 x 8 +4 %, the larger workloads above; figures of the tile solver).  The
+// march's whole-device rounds gain more (201x201x101 x 16: FP64 73.5 -> 57.7 ms, FP32 59.0 -> 44.5, FP64
+// gradient 92.4 -> 76.9), one workgroup per source nothing (600x400 x 256: 14.4 either way), and a lower
+// line no more than the runs differ (60x75x75 sphere x 24 gradient, 2 x 2^22: 15.6 -> 15.4).  Results do not depend on
 // the split: every source is solved on its own, and a gradient's sums and its source-to-source
 // carry-over run over both halves in source order.
 constexpr int64_t kSplitNodes = (int64_t)3 << 22;
