@@ -966,7 +966,10 @@ __global__ void __launch_bounds__(256) k_march_finish(const InstDev* __restrict_
 
 static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-constexpr int kRoundBlocks = 512;  // blocks of a round over all instances: two per CU, all resident
+// Blocks of a round over all instances: two per CU, all resident (256 registers a lane).  Milliseconds at 256 /
+// 384 / 512 / 768 / 1024 blocks: 60x75x75 sphere x 24 gradient 17.5 / 16.4 / 15.4 / 17.5 / 17.7, 120x150x150
+// sphere x 32 - / - / 83.8 / 91.8 / 98.8, 201x201x101 x 16 60.3 / 59.4 / 58.4 (64 an instance from there on).
+constexpr int kRoundBlocks = 512;
 static int round_blocks(int ninst) { return std::max(1, std::min(kMaxBlocks, kRoundBlocks / std::max(1, ninst))); }
 
 // Bytes of the march's buffers: values, slowness, three pending buffers, own, two lists.
