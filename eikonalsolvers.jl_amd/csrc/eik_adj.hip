@@ -972,7 +972,7 @@ static int adj_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, int64_t nti
     // the last round's list length; none listed means converged (a round with nothing listed wakes
     // nothing, so every later round is empty too).
     CK(hipMemsetAsync(d_cnt, 0, kAdjWords * sizeof(unsigned), st));
-    k_fill_u32<<<nb(2 * (int64_t)ninst, 256), 256, 0, st>>>(W, 2 * (int64_t)ninst, 0u);
+    fill<unsigned>(st, W, 2 * (int64_t)ninst, 0u);
     const unsigned bx = nb(most, kSelectThreads);
     k_adj_select<<<bx * (unsigned)ninst, kSelectThreads, 0, st>>>(flags, apend, bx, d_inst, W + ninst, W, (int64_t*)list.p, d_cnt + kAdjSlots, true);
     FimStats stt{};

@@ -795,11 +795,6 @@ __global__ void __launch_bounds__(BS) k_band_select(unsigned* __restrict__ flags
     }
 }
 
-__global__ void k_fill_u32(unsigned* __restrict__ p, int64_t n, unsigned v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 __global__ void k_slowness(const double* __restrict__ vel, double* __restrict__ s64, float* __restrict__ s32,
                            int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1100,7 +1095,7 @@ static int fim_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, int64_t nti
     unsigned* W = (unsigned*)wm.p;      // 3 x ninst lowest pending values, by round mod 3
     unsigned* SL = d_cnt + kCntSlots;   // 3 round slots (list length, cursor), by round mod 3
     // round 0's lowest pending values from the seeded tiles; the other two buffers start empty
-    k_fill_u32<<<nblocks(3 * (int64_t)ninst, 256), 256, 0, st>>>(W, 3 * (int64_t)ninst, 0x7f800000u);
+    fill<unsigned>(st, W, 3 * (int64_t)ninst, 0x7f800000u);
     k_band_min<kSB><<<nblocks(ntiles, kSB), kSB, 0, st>>>(flags, pend, ntiles, d_inst, ninst, W,
                                                                       d_cnt + kCntFlagged);
     CK(hipGetLastError());
@@ -1150,10 +1145,10 @@ static int fim_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, int64_t nti
             // to reach the exact fixed point: nothing to verify
             if (settle > T(0)) break;
             if (verifying && h_cnt[kCntRounds] <= rounds_at_verify + 1u) break;  // verified
-            k_fill_u32<<<nblocks(ntiles, 256), 256, 0, st>>>(flags, ntiles, kFullBit);
-            k_fill_u32<<<nblocks(ntiles, 256), 256, 0, st>>>(pend, ntiles, 0u);
+            fill<unsigned>(st, flags, ntiles, kFullBit);
+            fill<unsigned>(st, pend, ntiles, 0u);
             // every tile now pends at 0: the next round's lowest pending value
-            k_fill_u32<<<nblocks(ninst, 256), 256, 0, st>>>(W + (size_t)(round % 3) * ninst, ninst, 0u);
+            fill<unsigned>(st, W + (size_t)(round % 3) * ninst, ninst, 0u);
             CK(hipGetLastError());
             verifying = true;
             rounds_at_verify = h_cnt[kCntRounds];
@@ -1459,11 +1454,11 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     if (!march) {
         // the tile solver's key pools start as an unreached node's key (+inf, -inf)
         if (f32) {
-            k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)kc.p, totN, EIK_INFF);
-            k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)sc.p, totN, -EIK_INFF);
+            fill<float>(st, kc.p, totN, EIK_INFF);
+            fill<float>(st, sc.p, totN, -EIK_INFF);
         } else {
-            k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)kc.p, totN, EIK_INF);
-            k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)sc.p, totN, -EIK_INF);
+            fill<double>(st, kc.p, totN, EIK_INF);
+            fill<double>(st, sc.p, totN, -EIK_INF);
         }
     }
     DevBuf& aflags = ctx->buf("fim_flags");  // adjoint rounds, one byte per adjoint tile
@@ -1478,15 +1473,15 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
         if (flags.ensure((size_t)maxt * sizeof(unsigned)) || pend.ensure((size_t)maxt * sizeof(unsigned)))
             return ctx->fail(EIK_ENOMEM, "out of device memory (tile flags)");
         CK(hipMemsetAsync(flags.p, 0, (size_t)maxt * sizeof(unsigned), st));
-        k_fill_u32<<<nblocks(maxt, 256), 256, 0, st>>>((unsigned*)pend.p, maxt, 0x7f800000u);
+        fill<unsigned>(st, pend.p, maxt, 0x7f800000u);
     }
 
     // coarse grids start at +inf (a march writes every node at its end)
     if (march) {
     } else if (prec != EIK_PREC_FP32)
-        k_fill<double><<<nblocks(totN, 256), 256, 0, st>>>((double*)ttc.p, totN, EIK_INF);
+        fill<double>(st, ttc.p, totN, EIK_INF);
     else
-        k_fill<float><<<nblocks(totN, 256), 256, 0, st>>>((float*)ttc.p, totN, EIK_INFF);
+        fill<float>(st, ttc.p, totN, EIK_INFF);
 
     std::vector<CornerDev> corners;
     // the march's init nodes: the source-box corners, or the points transferred from the refined box
@@ -1522,8 +1517,8 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
             return ctx->fail(EIK_ENOMEM, "out of device memory (refined grids)");
         CK(hipMemsetAsync(df.p, 0, (size_t)nfine_pts, st));
         if (!march_f) {
-            k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)kf.p, nfine_pts, EIK_INF);
-            k_fill<double><<<nblocks(nfine_pts, 256), 256, 0, st>>>((double*)sf.p, nfine_pts, -EIK_INF);
+            fill<double>(st, kf.p, nfine_pts, EIK_INF);
+            fill<double>(st, sf.p, nfine_pts, -EIK_INF);
         }
         const TTPools fpools{ttf.p, kf.p, sf.p, (uint8_t*)df.p};
         CK(hipMemcpyAsync(dfi.p, finst.data(), finst.size() * sizeof(InstDev), hipMemcpyHostToDevice, st));

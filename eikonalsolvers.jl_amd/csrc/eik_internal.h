@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/eik.h"
+#include "eik_launch.h"
 #include "eik_spans.h"
 #include "eik_stencil.h"
 
@@ -553,12 +554,14 @@ int gradient_total(eik_ctx* ctx, eik_model* M, const eik_params* P, int whichgra
                    const int64_t* rec_off, int64_t nsrc, double* gradvel, double* misf);
 int gradient_solve(eik_ctx* ctx, eik_model* M, const SourceSet& S, const eik_params* P, int whichgrad,
                    const double* pickobs, const double* stdobs, double* gradvel, double* gradsrc, double* misf);
-// fill kernel (eik_fim.hip), also used by the adjoint rounds
-__global__ void k_fill_u32(unsigned* __restrict__ p, int64_t n, unsigned v);
+// n elements from p on set to v, on the context's stream (fill_blocks)
 template <typename T>
-__global__ void k_fill(T* __restrict__ p, int64_t n, T v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+__global__ void __launch_bounds__(kFillThreads) k_fill(T* __restrict__ p, int64_t n, T v) {
+    for (int64_t i = (int64_t)blockIdx.x * kFillThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kFillThreads) p[i] = v;
+}
+template <typename T>
+inline void fill(hipStream_t st, void* p, int64_t n, T v) {
+    k_fill<T><<<fill_blocks(n), kFillThreads, 0, st>>>((T*)p, n, v);
 }
 struct FimStats {
     int64_t rounds = 0;        // solver rounds (one launch each)

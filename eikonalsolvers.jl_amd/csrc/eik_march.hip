@@ -964,8 +964,6 @@ __global__ void __launch_bounds__(256) k_march_finish(const InstDev* __restrict_
 
 // ================================================================= host side
 
-static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
-
 // Blocks of a round over all instances: two per CU, all resident (256 registers a lane).  Milliseconds at 256 /
 // 384 / 512 / 768 / 1024 blocks: 60x75x75 sphere x 24 gradient 17.5 / 16.4 / 15.4 / 17.5 / 17.7, 120x150x150
 // sphere x 32 - / - / 83.8 / 91.8 / 98.8, 201x201x101 x 16 60.3 / 59.4 / 58.4 (64 an instance from there on).
@@ -1119,10 +1117,10 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     unsigned long long* d_c = (unsigned long long*)ctx->buf("march_cnt").p;
     unsigned long long* h = (unsigned long long*)ctx->h_small;
     const bool device = sz.mode == kMarchDevice;
-    k_fill<T><<<nblocks(nb, 256), 256, 0, st>>>(M.tt, nb, tinf_host<T>());
-    k_fill_u32<<<nblocks((device ? 3 : 1) * nb, 256), 256, 0, st>>>(pend, (device ? 3 : 1) * nb, kIdle);
-    if (device) k_fill_u32<<<nblocks(nb, 256), 256, 0, st>>>(M.less, nb, kIdle);
-    k_fill_u32<<<1, 256, 0, st>>>((unsigned*)d_c, 32, 0u);
+    fill<T>(st, M.tt, nb, tinf_host<T>());
+    fill<unsigned>(st, pend, (device ? 3 : 1) * nb, kIdle);
+    if (device) fill<unsigned>(st, M.less, nb, kIdle);
+    fill<unsigned>(st, d_c, 32, 0u);
     k_march_bricks<ND, T><<<dim3((unsigned)std::min<int64_t>(1024, (sz.most * 64 + 255) / 256), (unsigned)sz.nowners), 256, 0, st>>>(
         d_inst, sz.owners, slowpool, (T*)ctx->buf("march_slow").p);
     CK(hipGetLastError());
