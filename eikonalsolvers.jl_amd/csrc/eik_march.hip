@@ -627,7 +627,7 @@ constexpr int kRoundThreads = 256;
 constexpr int kRoundPer = 4;                                 // entries per thread and pass
 constexpr int kRoundPass = kRoundThreads * kRoundPer;        // entries a block looks at together
 constexpr int kRoundRun = 1024;                              // nodes a block runs per round; more wait
-constexpr int kRoundFresh = 3072;                            // newly listed nodes a block collects
+constexpr int kRoundFresh = 3072;                            // newly listed nodes a pass collects in LDS
 // a segment holds an equal part of the list, twice over, and what a block's wakes can add
 __host__ __device__ __forceinline__ unsigned seg_cap(unsigned nodes, unsigned blocks) {
     return 2u * (list_cap(nodes) / blocks) + 4096u;
@@ -821,6 +821,10 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         }
         lds_barrier();
         const unsigned nrun = min(s_nrun, (unsigned)kRoundRun), nkeep = s_nkeep;
+        const auto list_fresh = [&](unsigned j, unsigned l) {
+            if (j < scap) to[j] = l | kNoHint << kHintShift;
+            at<ND>(own, l) = blk * scap + j;
+        };
         for (unsigned b = done + (unsigned)(tid & ~63); b < nrun; b += kRoundThreads) {
             const unsigned j = b + lane;
             const bool on = j < nrun;
@@ -847,6 +851,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
 #pragma unroll
             for (int k = 0; k < 4 * ND; k++)
                 if (k < 2 * ND || two) total += (unsigned)__popcll(__ballot((fresh >> k) & 1u));
+            // a pass that runs a thousand nodes can list more than LDS holds: the rest goes to its place at once
             if (total) {
                 unsigned to_at = 0u;
                 if (lane == 0) to_at = atomicAdd(&s_nfresh, total);
@@ -856,7 +861,10 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
                     if (k < 2 * ND || two) {
                         const unsigned long long m = __ballot((fresh >> k) & 1u);
                         const unsigned f = to_at + lane_rank(m);
-                        if (((fresh >> k) & 1u) && f < (unsigned)kRoundFresh) s_fresh[f] = who[k];
+                        if ((fresh >> k) & 1u) {
+                            if (f < (unsigned)kRoundFresh) s_fresh[f] = who[k];
+                            else list_fresh(out + nkeep + f, who[k]);
+                        }
                         to_at += (unsigned)__popcll(m);
                     }
                 }
@@ -866,15 +874,11 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         lds_barrier();
         done = nrun;
         const unsigned nfresh = s_nfresh;
-        if (tid == 0 && (nfresh > (unsigned)kRoundFresh || out + nkeep + nfresh > scap)) atomicOr(&counters[3], kOverflow);
+        if (tid == 0 && out + nkeep + nfresh > scap) atomicOr(&counters[3], kOverflow);
         for (unsigned i = tid; i < nkeep; i += kRoundThreads)
             if (out + i < scap) to[out + i] = s_keep[i];
-        for (unsigned i = tid; i < min(nfresh, (unsigned)kRoundFresh); i += kRoundThreads) {
-            const unsigned j = out + nkeep + i;
-            if (j < scap) to[j] = s_fresh[i] | kNoHint << kHintShift;
-            at<ND>(own, s_fresh[i]) = blk * scap + j;
-        }
-        out = min(out + nkeep + min(nfresh, (unsigned)kRoundFresh), scap);
+        for (unsigned i = tid; i < min(nfresh, (unsigned)kRoundFresh); i += kRoundThreads) list_fresh(out + nkeep + i, s_fresh[i]);
+        out = min(out + nkeep + nfresh, scap);
     }
     lowest = wave_min_u32(lowest);
     if (lane == 0) {
