@@ -1289,7 +1289,7 @@ static double corner_dist(const InstDev& I, int nd, int kind, const int* ijk, co
     return distance2points(kind, nd, xyz, src);
 }
 
-// The whole solve again, by the tile solver (a march whose lists were too short).
+// The whole solve again, by the tile solver (a march that stopped short, kMarchAgain).
 static int solve_with_tiles(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
     ctx->tiles_only = true;
     const int rc = forward_solve(ctx, G, prec, P);
@@ -1557,7 +1557,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                        : fim_run(ctx, nd, EIK_PREC_FP64, kind, (const InstDev*)dfi.p, (int)nsrc, ntiles_f, fpools, slf.p,
                                  P->fast == 0, false, &fst);
         ctx->span_fine = false;
-        if (rc == kMarchOverflow) return solve_with_tiles(ctx, G, prec, P);
+        if (rc == kMarchAgain) return solve_with_tiles(ctx, G, prec, P);
         if (rc) return rc;
         ctx->stats[1] = tm.mark();
         ctx->stats[14] = fst.kernel_ms;
@@ -1628,7 +1628,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                                near, &cst)
                    : fim_run(ctx, nd, prec, kind, (const InstDev*)dci.p, (int)nsrc, ntiles_c, cpools, slow, P->fast == 0,
                              near, &cst);
-    if (rc == kMarchOverflow) return solve_with_tiles(ctx, G, prec, P);
+    if (rc == kMarchAgain) return solve_with_tiles(ctx, G, prec, P);
     if (rc) return rc;
     ctx->stats[2] = tm.mark();
     ctx->stats[4] = cst.activations;

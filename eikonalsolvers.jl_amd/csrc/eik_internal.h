@@ -587,6 +587,7 @@ struct TTPools {
 constexpr int kInitDepth = 0xff;
 struct MarchCtl {
     unsigned max_rounds, settle_round, settle_step;
+    unsigned list_limit;  // entries of a list (device rounds: of a block's segment) at most
     double settle_tol;
 };
 struct MarchSeeds {
@@ -612,7 +613,7 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
 int64_t march_request_bytes(const eik_grid& g, int64_t nsrc, const eik_params& P);
 // Device buffers for marches of these sizes; false if they do not fit.
 bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst);
-constexpr int kMarchOverflow = 1000;  // march_run: a list was too short (see list_cap)
+constexpr int kMarchAgain = 1000;  // march_run: a list was too short (list_cap), or no convergence
 MarchCtl march_ctl(const std::vector<InstDev>& inst);
 int march_run(eik_ctx* ctx, int nd, int prec, int kind, const InstDev* d_inst, int ninst, const MarchSize& sz,
               const TTPools& pools, const void* slowpool, const MarchSeeds& sd, bool exact, bool near, FimStats* fs);

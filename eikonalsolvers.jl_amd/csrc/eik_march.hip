@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
     const InstDev& I = inst[blockIdx.x];
     const GridView<ND, T> G = grid_view<ND, T>(I, pools, M);
     const unsigned nodes = 64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]);
-    const unsigned lcap = list_cap(nodes);
+    const unsigned lcap = min(list_cap(nodes), ctl.list_limit);
     unsigned* const sp = inst_lists(M, I, blockIdx.x);  // list k's entries beyond kGroupList: sp + k * lcap
     unsigned* const pend = M.p[0] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
@@ -621,6 +621,7 @@ struct MarchSlots {
     unsigned* low;   // the same: lowest pending value among them
     unsigned* ran;   // per block: count, then up to kRoundRun nodes
     unsigned* stat;  // per block: nodes replayed and changed
+    unsigned limit;  // entries of a segment at most (MarchCtl::list_limit)
 };
 constexpr int kMaxBlocks = 64;                               // per instance: a wave scans their words
 constexpr int kRoundThreads = 256;
@@ -641,7 +642,7 @@ __global__ void __launch_bounds__(256) k_march_seed(const InstDev* __restrict__ 
     const int in = blockIdx.x;
     const InstDev& I = inst[in];
     const GridView<ND, T> G = grid_view<ND, T>(I, pools, M);
-    const unsigned scap = seg_cap(64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]), blocks);
+    const unsigned scap = min(seg_cap(64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]), blocks), S.limit);
     unsigned* const list = inst_lists(M, I, in);
     unsigned* const pend = M.p[0] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
@@ -703,7 +704,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
     unsigned* const pr = M.p[rslot] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
     unsigned* const less = M.less + I.tile_base * 64;
-    const unsigned scap = seg_cap(nodes, nblk), half = scap * nblk;  // a list: nblk segments
+    const unsigned scap = min(seg_cap(nodes, nblk), S.limit), half = scap * nblk;  // a list: nblk segments
     const unsigned* const from = inst_lists(M, I, in) + (par ? half : 0u);
     unsigned* const to = inst_lists(M, I, in) + (par ? 0u : half) + (size_t)blk * scap;
     const unsigned end = wave_scan(c0), cnt = (unsigned)__builtin_amdgcn_readlane((int)end, 63);
@@ -1085,13 +1086,18 @@ MarchCtl march_ctl(const std::vector<InstDev>& inst) {
     const int64_t r = std::min<int64_t>(2000 + 50 * len, 1 << 26);
     c.settle_round = (unsigned)(es ? std::max(0, atoi(es)) : r);
     c.settle_step = (unsigned)(r / 4);
-    c.max_rounds = (unsigned)(20 * r + 50000);
+    // by then the tolerance has passed every change (1e-12 x 10^20), whatever circulates
+    c.max_rounds = (unsigned)(6 * r);
+    const char* el = getenv("EIK_LIST_LIMIT");  // test hook: lists of at most this many entries
+    c.list_limit = el ? (unsigned)std::max(1, atoi(el)) : 0xffffffffu;
     return c;
 }
 
-// nodes still listed over the instances (next round's slot), for the host
+// For the host: bit 0 if some instance has nodes listed (next round's slot), kOverflow if a list was too
+// short.  After an overflow some pending nodes are in no list and hold up others for good, so the march
+// has to end there.
 __global__ void __launch_bounds__(256) k_march_left(const unsigned* __restrict__ cnt, int ninst,
-                                                    unsigned long long* __restrict__ left) {
+                                                    const unsigned long long* __restrict__ counters, unsigned long long* __restrict__ left) {
     __shared__ unsigned s_any;
     if (threadIdx.x == 0) s_any = 0u;
     __syncthreads();
@@ -1099,7 +1105,7 @@ __global__ void __launch_bounds__(256) k_march_left(const unsigned* __restrict__
     for (int i = threadIdx.x; i < ninst; i += 256) any |= cnt[i];
     if (any) s_any = 1u;
     __syncthreads();
-    if (threadIdx.x == 0) *left = s_any;
+    if (threadIdx.x == 0) *left = s_any | (counters[3] & kOverflow);
 }
 
 template <typename T>
@@ -1143,7 +1149,7 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
         unsigned* words = (unsigned*)(d_c + 32);
         const int blocks = round_blocks(ninst);
         const size_t nw = (size_t)kMaxBlocks * ninst;
-        const MarchSlots S{words, words + 2 * nw, (unsigned*)ctx->buf("march_ran").p, words + 4 * nw};
+        const MarchSlots S{words, words + 2 * nw, (unsigned*)ctx->buf("march_ran").p, words + 4 * nw, ctl.list_limit};
         const dim3 gr((unsigned)ninst, (unsigned)blocks);
         k_march_seed<ND, T><<<(unsigned)ninst, 256, 0, st>>>(d_inst, ninst, P, M, sd.seeds, sd.cap, sd.nseed, S, blocks, d_c);
         CK(hipGetLastError());
@@ -1162,14 +1168,15 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
                 CK(hipGetLastError());
             }
             const int k = (int)(batch & 1);
-            k_march_left<<<1, 256, 0, st>>>(S.cnt + (size_t)par * nw, (int)nw, d_c + 4 + k);
+            k_march_left<<<1, 256, 0, st>>>(S.cnt + (size_t)par * nw, (int)nw, d_c, d_c + 4 + k);
             CK(hipMemcpyAsync(h + 16 + k, d_c + 4 + k, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
             CK(hipEventRecord(ctx->kev[2 + k], st));
             if (batch > 0) {
                 CK(hipEventSynchronize(ctx->kev[2 + (k ^ 1)]));
+                if (h[16 + (k ^ 1)] & kOverflow) return kMarchAgain;
                 if (h[16 + (k ^ 1)] == 0ull) break;
             }
-            if (rounds >= ctl.max_rounds) return ctx->fail(EIK_ENOCONV, "traveltime solve did not converge");
+            if (rounds >= ctl.max_rounds) return kMarchAgain;
         }
         k_march_stats<<<std::max(1, ninst * blocks / 2048), 256, 0, st>>>(S.stat, ninst * blocks, d_c);
         CK(hipGetLastError());
@@ -1180,8 +1187,7 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     CK(hipGetLastError());
     CK(hipMemcpyAsync(h, d_c, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     CK(hipStreamSynchronize(st));
-    if (h[3] & kOverflow) return kMarchOverflow;
-    if (h[3]) return ctx->fail(EIK_ENOCONV, "traveltime solve did not converge");
+    if (h[3]) return kMarchAgain;
     FimStats s{};
     float ms = 0.f;
     CK(hipEventElapsedTime(&ms, ctx->kev[0], ctx->kev[1]));

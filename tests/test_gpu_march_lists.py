@@ -1,12 +1,56 @@
-"""A device round of the ordered march that lists more nodes than its LDS buffer holds (3072 a block)
-loses none of them: the tile solver's bits in FP64."""
+"""Lists of the ordered march at their limits.  A march whose lists are too short stops and the call is
+solved by the tile solver (EIK_LIST_LIMIT shortens them here); a device round that lists more nodes
+than its LDS buffer holds (3072 a block) loses none of them.  In FP64 both ways end at the tile
+solver's bits."""
+import time
+
 import numpy as np
 import pytest
 
+import cases
 from eikonalsolvers.grids import ExtraParams
 from eikonalsolvers.synthetic import c5_request
+from test_zz_no_alloc import _call
 
 pytestmark = pytest.mark.gpu
+
+MODELS = {
+    "cart2d": lambda: cases.random2d(seed=31, n=(70, 61), nsrc=3),
+    "cart3d": lambda: cases.random3d(seed=32, n=(25, 22, 19), nsrc=3),
+    "sphere2d": cases.sphere2d,
+    "sphere3d": cases.sphere3d,
+}
+
+
+@pytest.mark.parametrize("refine", [False, True])
+@pytest.mark.parametrize("kind", sorted(MODELS))
+def test_short_lists_end_on_the_tile_solver(eik, monkeypatch, kind, refine):
+    if kind == "sphere3d" and refine:
+        pytest.skip("3D spheres have no refinement")
+    grd, vel, src, recs = MODELS[kind]()
+    ep = ExtraParams(refinearoundsrc=refine)
+    monkeypatch.setenv("EIK_MARCH", "0")
+    _, t0 = eik.eiktraveltime(vel, grd, src, recs, returntt=True, extraparams=ep)
+    model = eik.EikModel(vel, grd)
+    for mode in (1, 2):
+        monkeypatch.setenv("EIK_MARCH", str(mode))
+        for limit in (1, 30):  # the seeds alone, and a front some rounds on
+            monkeypatch.setenv("EIK_LIST_LIMIT", str(limit))
+            print(f"short lists {kind} refine={refine} mode={mode} limit={limit}", flush=True)
+            at = time.perf_counter()
+            _, t = eik.eiktraveltime(vel, grd, src, recs, returntt=True, extraparams=ep)
+            took = time.perf_counter() - at
+            st = eik.default_context().last_stats()
+            for s in range(len(src)):
+                assert np.array_equal(t[s], t0[s]), (mode, limit, s)
+            if limit == 1 or mode == 1:  # (segments of 30 entries are enough for the smallest grids)
+                assert st["verify_rounds"] >= 1, "the tile solver did not run"
+            assert took < 1.0, "the march went on after its lists had overflowed"
+            rc0, p0, g0 = _call("eik_traveltime", model, src, recs, ep, True)
+            rc1, p1, g1 = _call("eik_traveltime_noalloc", model, src, recs, ep, True)
+            assert rc0 == 0 and rc1 == 0
+            assert np.array_equal(p1, p0) and np.array_equal(g1, g0), (mode, limit)
+    model.close()
 
 
 def test_more_newly_listed_nodes_than_a_round_collects(eik, monkeypatch):
