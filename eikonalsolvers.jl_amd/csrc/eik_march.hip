@@ -164,8 +164,9 @@ __device__ __forceinline__ bool quiet_change(T v0, T k0, T v1, T k1, T settle) {
     return fabs(v1 - v0) <= settle * v0 && fabs(k1 - k0) <= settle * fabs(k0);
 }
 
-// The pending value of a woken node, as bits: never 0 (may_run steps it down by one).
-__device__ __forceinline__ unsigned pend_bits(float p) { return max(__float_as_uint(p), 1u); }
+// The pending value of a woken node, as bits: never 0 (may_run steps it down by one), and never an
+// idle node's, whatever the expected value (times beyond the float range: its largest number).
+__device__ __forceinline__ unsigned pend_bits(float p) { return min(max(__float_as_uint(p), 1u), kIdle - 1u); }
 
 // Replays node l (on: this lane has one) and writes it if it changed; returns whether it did.
 // p: the round's pending values (only read here).  wake(k, w, q, idle, pq, p): if w, neighbour q (the
