@@ -395,7 +395,10 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 
 // Listing.  Several nodes of a round may wake the same idle node; each lists it and writes its own
 // list position into the node's `own` word, and the next selection drops the entries that the word
-// does not name.  No atomic's return value is waited for.
+// does not name.  No atomic's return value is waited for.  Where the writers are blocks of several XCDs
+// the word is written by an atomic: after two plain stores from two XCDs in one launch each XCD went on
+// reading its own in the next, so that both entries stood, and one of them stayed listed for good when
+// the node had run.
 
 // The neighbours of the init nodes (values in the x-fastest pool) are pending with their smallest init
 // neighbour's value: add(q, p) for each of them, by the threads of one block.  The init nodes'
@@ -823,9 +826,10 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         }
         lds_barrier();
         const unsigned nrun = min(s_nrun, (unsigned)kRoundRun), nkeep = s_nkeep;
+        // blocks on several XCDs may list a node in one round: an atomic (see "Listing" above)
         const auto list_fresh = [&](unsigned j, unsigned l) {
             if (j < scap) to[j] = l | kNoHint << kHintShift;
-            at<ND>(own, l) = blk * scap + j;
+            (void)__hip_atomic_exchange(&at<ND>(own, l), blk * scap + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         };
         for (unsigned b = done + (unsigned)(tid & ~63); b < nrun; b += kRoundThreads) {
             const unsigned j = b + lane;
