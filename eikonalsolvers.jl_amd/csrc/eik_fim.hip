@@ -1291,6 +1291,7 @@ static double corner_dist(const InstDev& I, int nd, int kind, const int* ijk, co
 
 // The whole solve again, by the tile solver (a march that stopped short, kMarchAgain).
 static int solve_with_tiles(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
+    if (getenv("EIK_VERBOSE")) fprintf(stderr, "libeik: march stopped short, solving with tiles\n");
     ctx->tiles_only = true;
     const int rc = forward_solve(ctx, G, prec, P);
     ctx->tiles_only = false;
@@ -1501,7 +1502,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     auto add_seed = [&](int64_t s, const InstDev& I, const int* g) {
         if (any_march) seedpt[(size_t)(s * kCorn + nseed[s]++)] = SrcPt{(int32_t)s, -1, g[0] + (int64_t)I.n[0] * (g[1] + (int64_t)I.n[1] * g[2])};
     };
-    MarchSeeds seeds{(const SrcPt*)dsp.p, kCorn, (const int*)dns.p, march_ctl(cinst)};
+    MarchSeeds seeds{(const SrcPt*)dsp.p, kCorn, (const int*)dns.p, march_ctl(cinst, finst)};
     if (P->refinearoundsrc) {
         DevBuf& dfi = ctx->buf("inst_fine");
         DevBuf& dfd = ctx->buf("fine_desc");

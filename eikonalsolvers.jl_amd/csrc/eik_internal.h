@@ -583,12 +583,11 @@ struct TTPools {
     uint8_t* d;
 };
 // Ordered marching (eik_march.hip).  Depth byte of an init node while a march runs; the init nodes of
-// every instance (cap entries each, `node` used); the settling stages and the limit, in rounds.
+// every instance (cap entries each, `node` used); the limit in rounds.
 constexpr int kInitDepth = 0xff;
 struct MarchCtl {
-    unsigned max_rounds, settle_round, settle_step;
+    unsigned max_rounds;
     unsigned list_limit;  // entries of a list (device rounds: of a block's segment) at most
-    double settle_tol;
 };
 struct MarchSeeds {
     const SrcPt* seeds;
@@ -613,8 +612,8 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
 int64_t march_request_bytes(const eik_grid& g, int64_t nsrc, const eik_params& P);
 // Device buffers for marches of these sizes; false if they do not fit.
 bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst);
-constexpr int kMarchAgain = 1000;  // march_run: a list was too short (list_cap), or no convergence
-MarchCtl march_ctl(const std::vector<InstDev>& inst);
+constexpr int kMarchAgain = 1000;  // march_run: a list was too short (list_cap), or the limit was reached (march_ctl)
+MarchCtl march_ctl(const std::vector<InstDev>& coarse, const std::vector<InstDev>& fine);
 int march_run(eik_ctx* ctx, int nd, int prec, int kind, const InstDev* d_inst, int ninst, const MarchSize& sz,
               const TTPools& pools, const void* slowpool, const MarchSeeds& sd, bool exact, bool near, FimStats* fs);
 double f32_settle();  // EIK_F32_SETTLE, EIK_MIX_SETTLE (eik_fim.hip)

@@ -157,7 +157,7 @@ __device__ __forceinline__ GridView<ND, T> grid_view(const InstDev& I, const TTP
 __device__ __forceinline__ double reach_key(double c) { return c; }
 __device__ __forceinline__ float reach_key(float c) { return c < EIK_INFF ? c - 2.f * kTieUlps * 1.1920929e-7f * fabsf(c) : c; }
 
-// A change smaller than `settle` relative (value and key) wakes nothing; see march_run.
+// A change smaller than `settle` relative (value and key) wakes nothing; see march_run_t.
 template <typename T>
 __device__ __forceinline__ bool quiet_change(T v0, T k0, T v1, T k1, T settle) {
     if (!(settle > T(0)) || !(v0 < tinf<T>())) return false;
@@ -533,11 +533,6 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
         // replay and wake
         const unsigned nrun = min(s_nrun[par], (unsigned)kGroupRun);
         if (tid == 0) s_nrun[par ^ 1] = 0u;
-        T stl = settle;
-        if (round >= ctl.settle_round) {
-            stl = (T)ctl.settle_tol;
-            for (unsigned r = ctl.settle_round + ctl.settle_step; r <= round; r += ctl.settle_step) stl *= T(10);
-        }
         for (unsigned b = (unsigned)(tid & ~63); b < nrun; b += BT) {
             const unsigned j = b + lane;
             const bool on = j < nrun;
@@ -545,7 +540,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
             unsigned who[4 * ND] = {}, fresh = 0u;
             bool two;
             const bool chg = relax_node<ND, T, SPH, MIX, NEAR>(
-                I, G, mcart, pend, l, on, stl, &two, [&](int k, bool w, unsigned q, bool idle, unsigned, float p) {
+                I, G, mcart, pend, l, on, settle, &two, [&](int k, bool w, unsigned q, bool idle, unsigned, float p) {
                     who[k] = q;
                     if (w) {
                         const unsigned pu = pend_bits(p);
@@ -1081,18 +1076,17 @@ bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) 
     return true;
 }
 
-// Settling starts after far more rounds than any converging march needs (measured: below 8 rounds
-// per grid node along the axes together), the tolerance growing tenfold every quarter of that.
-MarchCtl march_ctl(const std::vector<InstDev>& inst) {
+// The limit lies far above what a converging march needs (measured: up to 9 rounds per grid node along
+// the axes together).  A march that has not ended by then circulates among near-ties, or in an order
+// that means nothing (times that underflow a float), and the tile solver, which settles such cycles at
+// rounding level, takes the call over.
+MarchCtl march_ctl(const std::vector<InstDev>& coarse, const std::vector<InstDev>& fine) {
     int64_t len = 1;
-    for (const InstDev& I : inst) len = std::max(len, (int64_t)I.n[0] + I.n[1] + I.n[2]);
+    for (const std::vector<InstDev>* v : {&coarse, &fine})
+        for (const InstDev& I : *v) len = std::max(len, (int64_t)I.n[0] + I.n[1] + I.n[2]);
     MarchCtl c{};
-    const char* es = getenv("EIK_SETTLE_ROUND");  // test hook: settle from an earlier round
-    const int64_t r = std::min<int64_t>(2000 + 50 * len, 1 << 26);
-    c.settle_round = (unsigned)(es ? std::max(0, atoi(es)) : r);
-    c.settle_step = (unsigned)(r / 4);
-    // by then the tolerance has passed every change (1e-12 x 10^20), whatever circulates
-    c.max_rounds = (unsigned)(6 * r);
+    const char* es = getenv("EIK_SETTLE_ROUND");  // test hook: settle from an earlier round (the tile solver's)
+    c.max_rounds = (unsigned)(es ? std::max(0, atoi(es)) : std::min<int64_t>(2000 + 32 * len, 1 << 26));
     const char* el = getenv("EIK_LIST_LIMIT");  // test hook: lists of at most this many entries
     c.list_limit = el ? (unsigned)std::max(1, atoi(el)) : 0xffffffffu;
     return c;
@@ -1140,9 +1134,11 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
         d_inst, sz.owners, slowpool, (T*)ctx->buf("march_slow").p);
     CK(hipGetLastError());
     MarchCtl ctl = sd.ctl;
-    const T settle_tol = sizeof(T) == 8 ? T(1e-12) : T(4e-6);
-    ctl.settle_tol = (double)settle_tol;
-    const T settle = MIX ? T(mix_settle()) : (sizeof(T) == 8 ? (!exact ? settle_tol : T(0)) : T(f32_settle()));
+    // changes below this relative size wake nothing (as in the tile solver; 0 in an exact solve)
+    const T settle = MIX ? T(mix_settle()) : (sizeof(T) == 8 ? (!exact ? T(1e-12) : T(0)) : T(f32_settle()));
+    const int blocks = round_blocks(ninst);
+    // (march_ctl's limit, and rounds for the nodes that a round has no room for)
+    if (ctl.max_rounds) ctl.max_rounds += (unsigned)(4 * sz.most * 64 / (device ? (int64_t)kRoundRun * blocks : (int64_t)kGroupRun));
     CK(hipEventRecord(ctx->kev[0], st));
     int64_t rounds = 0;
     if (!device) {
@@ -1152,7 +1148,6 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
         CK(hipGetLastError());
     } else {
         unsigned* words = (unsigned*)(d_c + 32);
-        const int blocks = round_blocks(ninst);
         const size_t nw = (size_t)kMaxBlocks * ninst;
         const MarchSlots S{words, words + 2 * nw, (unsigned*)ctx->buf("march_ran").p, words + 4 * nw, ctl.list_limit};
         const dim3 gr((unsigned)ninst, (unsigned)blocks);
@@ -1161,14 +1156,9 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
         int par = 0;  // the list the next round reads
         // two batches are in flight: the host looks at what the one before left while the next runs
         for (int64_t batch = 0;; batch++) {
-            T stl = settle;
-            if (rounds >= ctl.settle_round) {
-                stl = settle_tol;
-                for (int64_t r = (int64_t)ctl.settle_round + ctl.settle_step; r <= rounds; r += ctl.settle_step) stl *= T(10);
-            }
             for (int r = 0; r < kMarchBatch; r++, rounds++) {
                 const int slot = (int)(rounds % 3);
-                k_march_round<ND, T, SPH, MIX, NEAR><<<gr, kRoundThreads, 0, st>>>(d_inst, ninst, P, M, S, slot, par, stl, d_c);
+                k_march_round<ND, T, SPH, MIX, NEAR><<<gr, kRoundThreads, 0, st>>>(d_inst, ninst, P, M, S, slot, par, settle, d_c);
                 par ^= 1;
                 CK(hipGetLastError());
             }
@@ -1209,7 +1199,6 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     s.rounds = device ? rounds : (int64_t)h[2];
     s.activations = s.updates / 64.0;
     s.sweeps = s.activations;
-    if (s.rounds > ctl.settle_round) s.settled = (int)(1 + (s.rounds - ctl.settle_round) / ctl.settle_step);
     if (fs) *fs = s;
     return EIK_OK;
 }
