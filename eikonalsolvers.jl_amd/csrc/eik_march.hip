@@ -992,20 +992,31 @@ static void march_bytes(int64_t ntiles, int64_t stiles, int64_t most, int ninst,
 // about the same for one instance as for one per CU, and grows with the instance's nodes; the
 // whole-device rounds cost about 12 us each whatever they hold, until the device is full; the tile
 // solver needs fewer, longer rounds, which wins where its sweeps are cheap and instances few and large.
-// Milliseconds per call, tiles / workgroup / device:
+// Milliseconds per call, tiles / workgroup / device, on a velocity that grows with depth (where two are
+// given, the second on layers):
 //   2D FP64   300x240 x 1   6.5 /  4.1 /  8.5    600x480 x 64   37.5 / 11.3 / 22.0
-//             1200x960 x 1  37.8 / 36.5 / 34.5   1200x960 x 4   52.8 / 38.7 / 34.1   1200x960 x 16 93.4 / 44.1 / 42.9
+//             900x890 x 4     - / 33 / 41        1100x900 x 16     - / 46 / 55, - / 37 / 43
+//             1200x960 x 4  52.8 / 38.7 / 34.1   1500x1400 x 24    - / 102 / 111, - / 87 / 83
+//             1700x1360 x 32 189 / 114 / 128, 163 / 100 / 93       2400x1920 x 32 342 / 251 / 207
+//             2400x1920 x 64   - / 264 / 288, - / 231 / 202        3000x2400 x 128  - / 516 / 631
 //             2400x1920 x 4 175 / 206 / 98       600x600 sphere x 8 50.8 / 28.2 / 31.2 (mixed the same)
-//   2D mixed  600x480 x 1   9.3 /  8.9 / 14.5    1200x960 x 4   29.4 / 38.2 / 33.3   1200x960 x 16 48.5 / 43.9 / 42.1
-//   2D FP32   300x240 x 1   4.5 /  3.6 /  8.4    600x480 x 4     9.3 /  9.4 / 16.0   600x480 x 16  14.5 /  9.8 / 15.6
-//             1200x960 x 16 36.9 / 42.8 / 43.8
+//   2D mixed  390x380 x 1   7.4 /  7.4, 7.0 / 6.1   570x560 x 1  11.7 / 13.4, 10.5 / 11.3
+//             570x560 x 4  14.0 / 14.3, 12.9 / 11.4 650x650 x 4  17.3 / 18.3, 16.1 / 14.2
+//             1060x1060 x 16 57 / 51 / 63, 62 / 45 / 48            1300x1300 x 16   73 / 82 / 85, 73 / 72 / 64
+//   2D FP32   300x300 x 1   4.8 /  5.0, 4.9 / 4.5   390x380 x 1   6.2 /  7.4, 5.9 / 5.9
+//             390x380 x 4   7.4 /  7.5, 7.5 / 6.2   450x450 x 4   8.8 /  9.8, 8.7 / 7.9
+//             640x620 x 8  17.6 / 17.6, 17.0 / 16.1 1200x960 x 16 36.9 / 42.8 / 43.8
 //   3D FP64   24^3 x 4      4.0 /  2.7 /  2.6    24^3 x 16       6.1 /  2.9 /  3.3   24^3 sphere x 1 1.5 / 1.2 / 1.7
 //             48x48x28 x 16 9.7 /  5.4 /  4.6    48x48x28 x 64  15.7 /  6.2 /  6.8   64x64x38 x 64  23.3 / 11.9 / 10.8
 //             100x100x60 x 1 11.3 / 32 / 6.7     200x200x120 x 4 74.6 / 1032 / 29.6 (mixed 54.2 / - / 28.9)
-//   3D FP32   48x48x28 x 1  3.5 /  4.5 /  3.9    150x150x90 x 1 15.0 / - / 12.2      150x150x90 x 16 33.0 / - / 26.2
-//             200x200x120 x 1 20.9 / - / 20.6    200x200x120 x 4 29.2 / - / 25.8     201x201x101 x 16 48.9 / - / 44.4
+//             140x140x100 x 200 288 / - / 278 (mixed 282 / - / 282)
+//   3D FP32   48x48x28 x 1  3.5 /  4.5 /  3.9    180x180x170 x 1 21.4 / - / 20.2     200x200x145 x 2 27.4 / - / 22.3
+//             240x240x140 x 4 40.1 / - / 38.7    260x260x150 x 4 46.8 / - / 47.5     260x260x150 x 8 64.5 / - / 57.1
+//             300x300x160 x 2 41.7 / - / 52.2    320x320x160 x 8 89 / - / 89         201x201x101 x 16 48.9 / - / 46
+//   (FP32 on a model of sharp diagonal stripes, 2.0 and 3.5: 120x120x60 x 4 22.9 / - / 30.3, 220x220x120 x 4 49 /
+//   - / 95: the size does not tell, and tiles take 1700 ms on noise where the march takes 30)
 // FP32 spheres stay with the tiles: within FP32 resolution their many near-ties have several fixed points,
-// and the march can circulate among them until it settles (600x600 x 8: 31 ms, the march 579).
+// and the march can circulate among them (600x600 x 8: 31 ms, the march 579).
 MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles, int64_t most, int ninst, int nowners) {
     const bool f32 = prec == EIK_PREC_FP32, sph = kind == EIK_GRID2D_SPHERE || kind == EIK_GRID3D_SPHERE;
     MarchSize z{ntiles, stiles, most, f32 ? sizeof(float) : sizeof(double), nullptr, nowners, kMarchNone};
@@ -1013,18 +1024,18 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
         z.mode = std::max(0, std::min(2, atoi(e)));
         return z;
     }
-    const int64_t nodes = most * 64;
+    const int64_t nodes = most * 64, n = ninst;
     if (f32 && sph) return z;
     if (nd == 2 && f32)
-        z.mode = nodes <= 150000 || (nodes <= 400000 && ninst >= 8) ? kMarchGroup : kMarchNone;
+        z.mode = nodes <= (n >= 8 ? 400000 : n >= 4 ? 150000 : 100000) ? kMarchGroup : kMarchNone;
     else if (nd == 2 && prec == EIK_PREC_MIXED && !sph)
-        z.mode = nodes <= 320000 || (nodes <= 1200000 && ninst >= 16) ? kMarchGroup : kMarchNone;
+        z.mode = nodes <= (n >= 16 ? 1200000 : n >= 4 ? 320000 : 210000) ? kMarchGroup : kMarchNone;
     else if (nd == 2)
-        z.mode = nodes <= 800000 || ninst >= 32 ? kMarchGroup : kMarchDevice;
-    else if (f32 && nodes > (ninst >= 4 ? 6000000 : 3000000))
+        z.mode = nodes <= std::max<int64_t>(800000, 70000 * n) ? kMarchGroup : kMarchDevice;
+    else if (f32 && nodes > (n >= 8 ? 10000000 : 6000000))
         z.mode = kMarchNone;
     else
-        z.mode = nodes <= std::max<int64_t>(16000, 1500 * (int64_t)ninst) ? kMarchGroup : kMarchDevice;
+        z.mode = nodes <= std::max<int64_t>(16000, 1500 * n) ? kMarchGroup : kMarchDevice;
     return z;
 }
 
