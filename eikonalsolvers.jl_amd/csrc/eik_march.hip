@@ -1017,6 +1017,13 @@ static void march_bytes(int64_t ntiles, int64_t stiles, int64_t most, int ninst,
 //   - / 95: the size does not tell, and tiles take 1700 ms on noise where the march takes 30)
 // FP32 spheres stay with the tiles: within FP32 resolution their many near-ties have several fixed points,
 // and the march can circulate among them (600x600 x 8: 31 ms, the march 579).
+// Unlike grids in one call (requests that share launches): the lines between the solvers hold for the largest
+// grid, and as many of them as the call's nodes make.  Device rounds give every instance the same number of
+// blocks, so the small ones' stand idle while the largest march on; beyond 1.5 M such bricks (nodes / 64) the
+// tiles are faster.  Tiles / device, idle bricks in M: 100^3 x 16 with 60^3 x 16 92 / 46 (0.2), 140^3 x 2 with
+// 80^3 x 10 and 60^3 x 25 111 / 81 (1.3), 120^3 x 10 with 90^3 x 100 210 / 200 (1.6), 112^3 x 31 with 73^3 x 51,
+// 83^3 x 53 and 68^3 x 56 228 / 341 (2.5), 157^3 x 9 with 68^3 x 56 190 / 256 (3.1), 222 of 68^3 to 157^3 308 / 841 (11).
+constexpr int64_t kIdleBricks = 1500000;
 MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles, int64_t most, int ninst, int nowners) {
     const bool f32 = prec == EIK_PREC_FP32, sph = kind == EIK_GRID2D_SPHERE || kind == EIK_GRID3D_SPHERE;
     MarchSize z{ntiles, stiles, most, f32 ? sizeof(float) : sizeof(double), nullptr, nowners, kMarchNone};
@@ -1024,7 +1031,7 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
         z.mode = std::max(0, std::min(2, atoi(e)));
         return z;
     }
-    const int64_t nodes = most * 64, n = ninst;
+    const int64_t nodes = most * 64, n = most > 0 ? (ntiles + most / 2) / most : 0;
     if (f32 && sph) return z;
     if (nd == 2 && f32)
         z.mode = nodes <= (n >= 8 ? 400000 : n >= 4 ? 150000 : 100000) ? kMarchGroup : kMarchNone;
@@ -1036,6 +1043,7 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
         z.mode = kMarchNone;
     else
         z.mode = nodes <= std::max<int64_t>(16000, 1500 * n) ? kMarchGroup : kMarchDevice;
+    if (z.mode == kMarchDevice && round_blocks(ninst) < kMaxBlocks && most * ninst - ntiles > kIdleBricks) z.mode = kMarchNone;
     return z;
 }
 

@@ -74,3 +74,18 @@ def test_more_newly_listed_nodes_than_a_round_collects(eik, monkeypatch):
     assert st["verify_rounds"] == 0 and st["node_updates"] < 2 * nodes, "the march did not solve the call itself"
     for m in models:
         m.close()
+
+
+def test_unlike_grids_in_one_call_take_the_faster_solver(eik):
+    """The same six grids go to the tile solver (the device rounds would leave most blocks idle beside the
+    largest grid's: 841 ms against 308); three grids of like size march."""
+    for ids, tiles in (((3, 10, 11, 23, 24, 28), True), ((10, 11, 24), False)):
+        reqs = [c5_request(i) for i in ids]
+        models = [eik.EikModel(r["vel"], r["grd"]) for r in reqs]
+        print("unlike grids " + ", ".join(f"{r['grd'].grsize}x{len(r['src'])}" for r in reqs), flush=True)
+        p = eik.traveltime_batch([(m, r["src"], r["recs"]) for r, m in zip(reqs, models)])
+        assert (eik.default_context().last_stats()["verify_rounds"] > 0) == tiles
+        for r, m, got in zip(reqs, models, p):
+            for a, b in zip(m.traveltime(r["src"], r["recs"]), got):
+                assert np.array_equal(a, b)
+            m.close()
