@@ -14,6 +14,7 @@
 
 #include "../../include/eik.h"
 #include "eik_launch.h"
+#include "eik_march_size.h"
 #include "eik_spans.h"
 #include "eik_stencil.h"
 
@@ -604,12 +605,13 @@ struct MarchSize {
     int nowners;
     int mode;  // kMarch*
 };
-// kMarchNone: the tile solver; kMarchGroup: one workgroup per instance; kMarchDevice: the whole device
-// per round
-constexpr int kMarchNone = 0, kMarchGroup = 1, kMarchDevice = 2;
 MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles, int64_t most, int ninst, int nowners);
-// bytes of the march's buffers in a request for nsrc sources on grid g (the tile solver needs none)
-int64_t march_request_bytes(const eik_grid& g, int64_t nsrc, const eik_params& P);
+// bytes of the march's buffers in one call for these grids' sources (the tile solver needs none)
+struct GridSet {
+    const eik_grid* g;
+    int64_t nsrc;
+};
+int64_t march_request_bytes(const std::vector<GridSet>& sets, const eik_params& P);
 // Device buffers for marches of these sizes; false if they do not fit.
 bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst);
 constexpr int kMarchAgain = 1000;  // march_run: a list was too short (list_cap), or the limit was reached (march_ctl)

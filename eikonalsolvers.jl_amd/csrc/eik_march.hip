@@ -117,18 +117,13 @@ struct MarchPools {
     unsigned* p[3];   // pending values
     unsigned* own;    // list position of a node's newest entry
     unsigned* less;   // a listed node's pending value lowered by a later wake (k_march_round)
-    unsigned* lists;  // two lists per instance (list_cap entries each)
+    unsigned* lists;  // two lists per instance (list_start)
 };
 
-// Entries a list is made for: every node once, and some of the duplicates that a round's wakes can
-// add (a list is a small part of the grid, apart from the smallest grids).  A march that needs more
-// than its lists hold reports it and is solved by the tile solver instead.
-__host__ __device__ __forceinline__ unsigned list_cap(unsigned nodes) { return nodes + nodes / 4u + 8192u; }
-constexpr int64_t kListSlack = 64 * 4096 + 64;  // seg_cap's constant part, over an instance's blocks
 constexpr unsigned long long kOverflow = 2ull;  // counters[3]: a list was too short (1: not converged)
 template <typename T>
-__device__ __forceinline__ unsigned* inst_lists(const MarchPools<T>& M, const InstDev& I, int in) {
-    return M.lists + 2 * (2 * (I.tile_base * 80 + (int64_t)in * 8192) + (int64_t)in * kListSlack);
+__device__ __forceinline__ unsigned* inst_lists(const MarchPools<T>& M, const InstDev& I, int in, int blocks) {
+    return M.lists + list_start(I.tile_base, in, blocks);
 }
 
 template <int ND, typename T>
@@ -449,7 +444,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
     const GridView<ND, T> G = grid_view<ND, T>(I, pools, M);
     const unsigned nodes = 64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]);
     const unsigned lcap = min(list_cap(nodes), ctl.list_limit);
-    unsigned* const sp = inst_lists(M, I, blockIdx.x);  // list k's entries beyond kGroupList: sp + k * lcap
+    unsigned* const sp = inst_lists(M, I, blockIdx.x, 0);  // list k's entries beyond kGroupList: sp + k * lcap
     unsigned* const pend = M.p[0] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -622,16 +617,10 @@ struct MarchSlots {
     unsigned* stat;  // per block: nodes replayed and changed
     unsigned limit;  // entries of a segment at most (MarchCtl::list_limit)
 };
-constexpr int kMaxBlocks = 64;                               // per instance: a wave scans their words
 constexpr int kRoundThreads = 256;
 constexpr int kRoundPer = 4;                                 // entries per thread and pass
 constexpr int kRoundPass = kRoundThreads * kRoundPer;        // entries a block looks at together
-constexpr int kRoundRun = 1024;                              // nodes a block runs per round; more wait
 constexpr int kRoundFresh = 3072;                            // newly listed nodes a pass collects in LDS
-// a segment holds an equal part of the list, twice over, and what a block's wakes can add
-__host__ __device__ __forceinline__ unsigned seg_cap(unsigned nodes, unsigned blocks) {
-    return 2u * (list_cap(nodes) / blocks) + 4096u;
-}
 
 template <int ND, typename T>
 __global__ void __launch_bounds__(256) k_march_seed(const InstDev* __restrict__ inst, int ninst, TTPools pools, MarchPools<T> M,
@@ -642,7 +631,7 @@ __global__ void __launch_bounds__(256) k_march_seed(const InstDev* __restrict__ 
     const InstDev& I = inst[in];
     const GridView<ND, T> G = grid_view<ND, T>(I, pools, M);
     const unsigned scap = min(seg_cap(64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]), blocks), S.limit);
-    unsigned* const list = inst_lists(M, I, in);
+    unsigned* const list = inst_lists(M, I, in, blocks);
     unsigned* const pend = M.p[0] + I.tile_base * 64;
     unsigned* const own = M.own + I.tile_base * 64;
     if (threadIdx.x == 0) {
@@ -704,8 +693,8 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
     unsigned* const own = M.own + I.tile_base * 64;
     unsigned* const less = M.less + I.tile_base * 64;
     const unsigned scap = min(seg_cap(nodes, nblk), S.limit), half = scap * nblk;  // a list: nblk segments
-    const unsigned* const from = inst_lists(M, I, in) + (par ? half : 0u);
-    unsigned* const to = inst_lists(M, I, in) + (par ? 0u : half) + (size_t)blk * scap;
+    const unsigned* const from = inst_lists(M, I, in, (int)nblk) + (par ? half : 0u);
+    unsigned* const to = inst_lists(M, I, in, (int)nblk) + (par ? 0u : half) + (size_t)blk * scap;
     const unsigned end = wave_scan(c0), cnt = (unsigned)__builtin_amdgcn_readlane((int)end, 63);
     s_end[wave][lane] = end;
     // this block's part of the list, a multiple of a wave's entries
@@ -969,24 +958,7 @@ __global__ void __launch_bounds__(256) k_march_finish(const InstDev* __restrict_
 
 // ================================================================= host side
 
-// Blocks of a round over all instances: two per CU, all resident (256 registers a lane).  Milliseconds at 256 /
-// 384 / 512 / 768 / 1024 blocks: 60x75x75 sphere x 24 gradient 17.5 / 16.4 / 15.4 / 17.5 / 17.7, 120x150x150
-// sphere x 32 - / - / 83.8 / 91.8 / 98.8, 201x201x101 x 16 60.3 / 59.4 / 58.4 (64 an instance from there on).
-constexpr int kRoundBlocks = 512;
-static int round_blocks(int ninst) { return std::max(1, std::min(kMaxBlocks, kRoundBlocks / std::max(1, ninst))); }
-
-// Bytes of the march's buffers: values, slowness, three pending buffers, own, two lists.
-static const char* const kMarchBuf[7] = {"march_tt", "march_slow", "march_pend", "march_own", "march_list", "march_cnt", "march_ran"};  // own: and less
-static void march_bytes(int64_t ntiles, int64_t stiles, int64_t most, int ninst, size_t esz, size_t* need) {
-    const size_t nb = (size_t)ntiles * 64;
-    need[0] = nb * esz;
-    need[1] = (size_t)stiles * 64 * esz;
-    need[2] = 3 * nb * sizeof(unsigned);
-    need[3] = 2 * nb * sizeof(unsigned);
-    need[4] = 2 * (2 * (nb + nb / 4 + 8192 * (size_t)ninst) + kListSlack * (size_t)ninst) * sizeof(unsigned);
-    need[5] = 256 + (4 * kMaxBlocks + 2 * (size_t)round_blocks(ninst)) * (size_t)ninst * sizeof(unsigned);
-    need[6] = (size_t)ninst * round_blocks(ninst) * (kRoundRun + 1) * sizeof(unsigned);
-}
+static const char* const kMarchBuf[kMarchBufs] = {"march_tt", "march_slow", "march_pend", "march_own", "march_list", "march_cnt", "march_ran"};
 
 // Which solver runs an instance set (EIK_MARCH overrides: kMarch*).  A workgroup per instance costs
 // about the same for one instance as for one per CU, and grows with the instance's nodes; the
@@ -1047,35 +1019,47 @@ MarchSize march_size(int nd, int kind, int prec, int64_t ntiles, int64_t stiles,
     return z;
 }
 
-int64_t march_request_bytes(const eik_grid& g, int64_t nsrc, const eik_params& P) {
-    eik_params e = effective_params(&P, g.kind);
-    const size_t esz = e.precision == EIK_PREC_FP32 ? 4 : 8;
-    InstDev I;
-    make_inst(g, I);
-    set_tiles(I, g.ndim);
-    const int64_t t = (int64_t)I.t[0] * I.t[1] * I.t[2];
-    size_t a[7], f[7] = {};
-    march_bytes(nsrc * t, t, t, (int)nsrc, esz, a);
-    if (e.refinearoundsrc) {
+int64_t march_request_bytes(const std::vector<GridSet>& sets, const eik_params& P) {
+    const eik_params e = effective_params(&P, sets[0].g->kind);
+    const int nd = sets[0].g->ndim, kind = sets[0].g->kind;
+    int64_t ntiles = 0, stiles = 0, most = 0, ninst = 0;
+    for (const GridSet& q : sets) {
+        InstDev I;
+        make_inst(*q.g, I);
+        set_tiles(I, nd);
+        const int64_t t = (int64_t)I.t[0] * I.t[1] * I.t[2];
+        ntiles += q.nsrc * t;
+        stiles += t;
+        most = std::max(most, t);
+        ninst += q.nsrc;
+    }
+    if (ninst == 0 || ninst > 65535) return 0;
+    const MarchSize z = march_size(nd, kind, e.precision, ntiles, stiles, most, (int)ninst, (int)sets.size());
+    size_t a[kMarchBufs], f[kMarchBufs] = {};
+    march_bytes(z.mode, ntiles, stiles, (int)ninst, z.esz, a);
+    if (e.refinearoundsrc) {  // (a box at the model's border is smaller, and may fall on the other side of a line)
         int64_t tf = 1;
-        for (int d = 0; d < g.ndim; d++)
-            tf *= ((2 * (int64_t)e.noderadius + 1) * e.downscalefactor + fwd_tile_edge(g.ndim)) / fwd_tile_edge(g.ndim);
-        march_bytes(nsrc * tf, nsrc * tf, tf, (int)nsrc, 8, f);
+        for (int d = 0; d < nd; d++)
+            tf *= ((2 * (int64_t)e.noderadius + 1) * e.downscalefactor + fwd_tile_edge(nd)) / fwd_tile_edge(nd);
+        for (int mode : {kMarchGroup, kMarchDevice}) {
+            size_t b[kMarchBufs];
+            march_bytes(mode, ninst * tf, ninst * tf, (int)ninst, 8, b);
+            for (int k = 0; k < kMarchBufs; k++) f[k] = std::max(f[k], b[k]);
+        }
     }
     int64_t b = 0;
-    for (int k = 0; k < 7; k++) b += (int64_t)std::max(a[k], f[k]);
+    for (int k = 0; k < kMarchBufs; k++) b += (int64_t)std::max(a[k], f[k]);
     return b + 65536;
 }
 
 bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) {
     if (ctx->tiles_only || ninst > 65535) return false;  // 65535: grid.y
-    size_t need[7] = {};
+    size_t need[kMarchBufs] = {};
     for (int i = 0; i < nsizes; i++) {
-        if (sizes[i].mode == kMarchNone) continue;
-        if (sizes[i].most * 64 >= (int64_t)kNodeMask) return false;
-        size_t n[7];
-        march_bytes(sizes[i].ntiles, sizes[i].stiles, sizes[i].most, ninst, sizes[i].esz, n);
-        for (int k = 0; k < 7; k++) need[k] = std::max(need[k], n[k]);
+        if (sizes[i].mode != kMarchNone && sizes[i].most * 64 >= (int64_t)kNodeMask) return false;
+        size_t n[kMarchBufs];
+        march_bytes(sizes[i].mode, sizes[i].ntiles, sizes[i].stiles, ninst, sizes[i].esz, n);
+        for (int k = 0; k < kMarchBufs; k++) need[k] = std::max(need[k], n[k]);
     }
     if (ctx->arena) {
         size_t sum = (size_t)ninst * 512 + 16384;
@@ -1083,11 +1067,11 @@ bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) 
         if (sum > ctx->arena->spare) return false;
     }
     int64_t grow = 0;
-    for (int k = 0; k < 7; k++)
+    for (int k = 0; k < kMarchBufs; k++)
         if (ctx->buf(kMarchBuf[k]).cap < need[k]) grow += (int64_t)(need[k] - ctx->buf(kMarchBuf[k]).cap);
     if (ctx->march_limit >= 0 && grow > ctx->march_limit) return false;
-    for (int k = 0; k < 7; k++)
-        if (ctx->buf(kMarchBuf[k]).ensure(need[k])) {
+    for (int k = 0; k < kMarchBufs; k++)
+        if (need[k] && ctx->buf(kMarchBuf[k]).ensure(need[k])) {
             (void)hipGetLastError();
             for (const char* b : kMarchBuf) ctx->buf(b).release();
             return false;
@@ -1141,7 +1125,7 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     unsigned* pend = (unsigned*)ctx->buf("march_pend").p;  // march_reserve made the buffers
     MarchPools<T> M{(T*)ctx->buf("march_tt").p, (const T*)ctx->buf("march_slow").p, {pend, pend + nb, pend + 2 * nb},
                     (unsigned*)ctx->buf("march_own").p, (unsigned*)ctx->buf("march_own").p + nb,
-                    (unsigned*)ctx->buf("march_list").p};
+                    (unsigned*)ctx->buf("march_list").p};  // (p[1], p[2] and less: device rounds alone)
     unsigned long long* d_c = (unsigned long long*)ctx->buf("march_cnt").p;
     unsigned long long* h = (unsigned long long*)ctx->h_small;
     const bool device = sz.mode == kMarchDevice;

@@ -244,11 +244,9 @@ static void worker(eik_server* S, int slot) {
         }
         // what the budget leaves beside the requests goes to the march's buffers, if they fit: with
         // less the call runs on the tile solver, so no request is held or refused for them
-        int64_t extra = 0;
-        for (int64_t k : ids) {
-            const eik_request& r = S->reqs[k].r;
-            extra += march_request_bytes(r.model->g, r.nsrc, r.params);
-        }
+        std::vector<GridSet> sets;
+        for (int64_t k : ids) sets.push_back(GridSet{&S->reqs[k].r.model->g, S->reqs[k].r.nsrc});
+        int64_t extra = march_request_bytes(sets, S->reqs[id].r.params);
         const int64_t room = S->budget_now - footprint_with(S, slot, std::max(bytes, S->held[slot]));
         if (extra > room) extra = 0;
         ctx->march_limit = extra;

@@ -89,3 +89,18 @@ def test_unlike_grids_in_one_call_take_the_faster_solver(eik):
             for a, b in zip(m.traveltime(r["src"], r["recs"]), got):
                 assert np.array_equal(a, b)
             m.close()
+
+
+def test_noalloc_marches_many_small_sources(eik):
+    """200 sources on a small grid fit the no-allocation block with the march's buffers."""
+    grd, vel, src, _ = cases.random2d(seed=51, n=(61, 44), nsrc=200)
+    recs = [src[:3] for _ in src]
+    ep = ExtraParams(refinearoundsrc=False)
+    model = eik.EikModel(vel, grd)
+    print("noalloc 61x44 x 200", flush=True)
+    rc0, p0, _ = _call("eik_traveltime", model, src, recs, ep, False)
+    rc1, p1, _ = _call("eik_traveltime_noalloc", model, src, recs, ep, False)
+    st = eik.default_context().last_stats()
+    assert rc0 == 0 and rc1 == 0 and np.array_equal(p0, p1)
+    assert st["verify_rounds"] == 0, "the tile solver solved it"
+    model.close()
