@@ -44,8 +44,8 @@ EIK_HD int64_t list_start(int64_t tile_base, int64_t in, int blocks) {
 
 // Bytes of the march's buffers for ninst instances of ntiles bricks in all and stiles bricks of slowness grids:
 // values, slowness, pending values, own words (and lowered values), lists, counters and segment words, run lists.
-// A workgroup per instance takes 26 bytes a node and 64 KB an instance (FP64, slowness included), device rounds
-// 56 and up to 4 MB.
+// In FP64 a workgroup per instance takes 26 bytes a node and 64 KB an instance, device rounds 48 and up to
+// 2.4 MB; a slowness grid 8 bytes a node of its model.
 constexpr int kMarchBufs = 7;
 inline void march_bytes(int mode, int64_t ntiles, int64_t stiles, int ninst, size_t esz, size_t* need) {
     const size_t nb = (size_t)ntiles * 64;

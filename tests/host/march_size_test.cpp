@@ -60,9 +60,9 @@ int main() {
     for (size_t n : none)
         if (n) return std::printf("the tile solver has march buffers\n"), 1;
     int bad = 0;
-    // a workgroup per source: 18 bytes a node beside the slowness, and 64 KB a source
-    bad += check("61x44 x 400", total(kMarchGroup, tiles(2, 61, 44, 1), 400, 8), 400 * (tiles(2, 61, 44, 1) * 64 * 26 + 65600) + 256);
-    bad += check("600x400 x 256", total(kMarchGroup, tiles(2, 600, 400, 1), 256, 8), 256 * (tiles(2, 600, 400, 1) * 64 * 26 + 65600) + 256);
+    // a workgroup per source: 26 bytes a node, 8 more for the one slowness grid, and 64 KB a source
+    bad += check("61x44 x 400", total(kMarchGroup, tiles(2, 61, 44, 1), 400, 8), 400 * (tiles(2, 61, 44, 1) * 64 * 26 + 65600) + tiles(2, 61, 44, 1) * 64 * 8 + 256);
+    bad += check("600x400 x 256", total(kMarchGroup, tiles(2, 600, 400, 1), 256, 8), 256 * (tiles(2, 600, 400, 1) * 64 * 26 + 65600) + tiles(2, 600, 400, 1) * 64 * 8 + 256);
     // device rounds: 48 bytes a node beside the slowness, and the segments' constants over 512 blocks
     bad += check("201x201x101 x 16", total(kMarchDevice, tiles(3, 201, 201, 101), 16, 8),
                  16 * tiles(3, 201, 201, 101) * 64 * 49 + (int64_t)(64 << 20));
