@@ -397,6 +397,20 @@ static eik_ctx* get_peer(eik_ctx* ctx) {
     return ctx->peer;
 }
 
+// A split call one of whose halves ran out of memory: the other half's march buffers can have been in its
+// way, whether they are still there or not.  True if the call is to run again, on tiles.
+static bool march_took_room(eik_ctx* ctx, int rc, int rc1) {
+    if (rc != EIK_ENOMEM && rc1 != EIK_ENOMEM) return false;
+    (void)march_release(ctx);
+    (void)march_release(ctx->peer);
+    return ctx->march_used || ctx->peer->march_used;
+}
+struct TilesOnly {
+    eik_ctx* c;
+    explicit TilesOnly(eik_ctx* ctx) : c(ctx) { c->tiles_only = c->peer->tiles_only = true; }
+    ~TilesOnly() { c->tiles_only = c->peer->tiles_only = false; }
+};
+
 // sources [a, b) of S, receivers re-based
 static SourceSet sub_sources(const SourceSet& S, int64_t a, int64_t b) {
     SourceSet T;
@@ -432,6 +446,7 @@ int eik_traveltime(eik_ctx* ctx, eik_model* model, int64_t nsrc, const double* c
     if (S.nrec() > 0 && !ttpicks) return ctx->fail(EIK_EINVAL, "null picks buffer");
     if (nsrc == 0) return EIK_OK;
     stats_begin(ctx);
+    MarchScope march(ctx);
     const bool split = ctx->split && nsrc >= 2 && nsrc * model->N >= kSplitNodes;
     eik_ctx* peer = split ? get_peer(ctx) : nullptr;
     if (!peer) {
@@ -457,10 +472,17 @@ int eik_traveltime(eik_ctx* ctx, eik_model* model, int64_t nsrc, const double* c
         rc1 = forward_solve(peer, model, S1, params->precision, params);
         if (rc1 == EIK_OK) rc1 = forward_picks(peer, model, S1, params->precision, picks1, grid1);
     };
-    std::thread th = start_thread(second);
-    rc = forward_solve(ctx, model, S0, params->precision, params);
-    if (rc == EIK_OK) rc = forward_picks(ctx, model, S0, params->precision, ttpicks, ttgrid);
-    finish_thread(th, second);
+    const auto both = [&] {
+        std::thread th = start_thread(second);
+        rc = forward_solve(ctx, model, S0, params->precision, params);
+        if (rc == EIK_OK) rc = forward_picks(ctx, model, S0, params->precision, ttpicks, ttgrid);
+        finish_thread(th, second);
+    };
+    both();
+    if (march_took_room(ctx, rc, rc1)) {
+        TilesOnly tiles(ctx);
+        both();
+    }
     if (rc) return rc;
     if (rc1) return ctx->fail(rc1, "%s", peer->err.c_str());
     merge_peer_stats(ctx);
@@ -494,6 +516,7 @@ int eik_traveltime_batch(eik_ctx* ctx, int32_t nreq, const eik_request* reqs) {
     if (G.empty()) return EIK_OK;
     const eik_params pe = effective_params(&reqs[0].params, reqs[0].model->g.kind);
     stats_begin(ctx);
+    MarchScope march(ctx);
     int rc = forward_solve(ctx, G, pe.precision, &pe);
     if (rc) return rc;
     std::vector<double> picks((size_t)std::max<int64_t>(nrec, 1));
@@ -568,6 +591,7 @@ int eik_gradient(eik_ctx* ctx, eik_model* model, int64_t nsrc, const double* coo
         return EIK_OK;
     }
     stats_begin(ctx);
+    MarchScope march(ctx);
     const bool split = ctx->split && nsrc >= 2 && nsrc * model->N >= kSplitNodes;
     eik_ctx* peer = split ? get_peer(ctx) : nullptr;
     if (!peer) {
@@ -592,9 +616,16 @@ int eik_gradient(eik_ctx* ctx, eik_model* model, int64_t nsrc, const double* coo
         rc1 = gradient_part(peer, model, S1, params, whichgrad, pickobs ? pickobs + r1 : nullptr,
                             stdobs ? stdobs + r1 : nullptr, gradsrc ? gradsrc + h * nd : nullptr, true, &parts[1]);
     };
-    std::thread th = start_thread(second);
-    rc = gradient_part(ctx, model, S0, params, whichgrad, pickobs, stdobs, gradsrc, false, &parts[0]);
-    finish_thread(th, second);
+    const auto both = [&] {
+        std::thread th = start_thread(second);
+        rc = gradient_part(ctx, model, S0, params, whichgrad, pickobs, stdobs, gradsrc, false, &parts[0]);
+        finish_thread(th, second);
+    };
+    both();
+    if (march_took_room(ctx, rc, rc1)) {
+        TilesOnly tiles(ctx);
+        both();
+    }
     if (rc) return rc;
     if (rc1) return ctx->fail(rc1, "%s", peer->err.c_str());
     merge_peer_stats(ctx);

@@ -1289,16 +1289,24 @@ static double corner_dist(const InstDev& I, int nd, int kind, const int* ijk, co
     return distance2points(kind, nd, xyz, src);
 }
 
-// The whole solve again, by the tile solver (a march that stopped short, kMarchAgain).
-static int solve_with_tiles(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
+static int forward_solve_once(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P);
+
+// A march that stopped short (kMarchAgain), or that left no room for what the call cannot do without: the
+// whole solve again, by the tile solver.
+int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
+    int rc = forward_solve_once(ctx, G, prec, P);
+    const bool marched = ctx->march_live;
+    ctx->march_live = false;
+    if (rc != kMarchAgain && !(rc == EIK_ENOMEM && marched && march_release(ctx))) return rc;
     if (getenv("EIK_VERBOSE")) fprintf(stderr, "libeik: march stopped short, solving with tiles\n");
+    const bool only = ctx->tiles_only;
     ctx->tiles_only = true;
-    const int rc = forward_solve(ctx, G, prec, P);
-    ctx->tiles_only = false;
+    rc = forward_solve_once(ctx, G, prec, P);
+    ctx->tiles_only = only;
     return rc;
 }
 
-int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
+static int forward_solve_once(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const eik_params* P) {
     const eik_model* M0 = G[0].M;
     const int nd = M0->g.ndim;
     const int kind = M0->g.kind;
@@ -1558,7 +1566,6 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                        : fim_run(ctx, nd, EIK_PREC_FP64, kind, (const InstDev*)dfi.p, (int)nsrc, ntiles_f, fpools, slf.p,
                                  P->fast == 0, false, &fst);
         ctx->span_fine = false;
-        if (rc == kMarchAgain) return solve_with_tiles(ctx, G, prec, P);
         if (rc) return rc;
         ctx->stats[1] = tm.mark();
         ctx->stats[14] = fst.kernel_ms;
@@ -1629,7 +1636,6 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
                                near, &cst)
                    : fim_run(ctx, nd, prec, kind, (const InstDev*)dci.p, (int)nsrc, ntiles_c, cpools, slow, P->fast == 0,
                              near, &cst);
-    if (rc == kMarchAgain) return solve_with_tiles(ctx, G, prec, P);
     if (rc) return rc;
     ctx->stats[2] = tm.mark();
     ctx->stats[4] = cst.activations;

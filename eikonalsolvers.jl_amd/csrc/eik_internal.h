@@ -7,6 +7,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -337,29 +338,10 @@ struct DevBuf {
     void* p = nullptr;
     size_t cap = 0;
     Arena* arena = nullptr;
-    int ensure(size_t n) {
-        if (n <= cap && p) return 0;
-        const size_t want = n ? n : 16;
-        if (arena) {
-            p = arena->carve(want);
-            cap = p ? want : 0;
-            return p ? 0 : -1;
-        }
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        cap = 0;
-        if (hipMalloc(&p, want) != hipSuccess) {
-            p = nullptr;
-            return -1;
-        }
-        cap = want;
-        return 0;
-    }
-    void release() {
-        if (p && !arena) (void)hipFree(p);
-        p = nullptr;
-        cap = 0;
-    }
+    eik_ctx* ctx = nullptr;
+    // 0, or -1 when there is no room, also without the march's buffers (unless a march is using them)
+    inline int ensure(size_t n);
+    inline void release();
 };
 
 // solver rounds enqueued between two host checks for convergence
@@ -404,6 +386,9 @@ struct eik_ctx {
     bool split = true;         // large calls may split their sources with the peer
     bool in_split = false;     // the current call is split (set on the context and its peer)
     int64_t march_limit = -1;  // bytes the march's buffers may grow by in this call (-1: no limit)
+    bool march_live = false;   // a march has its buffers (forward_solve)
+    bool march_used = false;   // march buffers have been held in this call (MarchScope)
+    std::atomic<int64_t> pooled{0};  // bytes of its own and its peer's buffers (kept by the owner)
     bool shared_device = false;  // other calls keep the device busy beside this one (see forward_solve)
     bool tiles_only = false;   // the tile solver instead of a march (see forward_solve)
     int xcap = 1;  // capacity per source of the transferred-point list
@@ -412,9 +397,9 @@ struct eik_ctx {
     Arena* arena = nullptr;
     std::map<std::string, DevBuf> abufs;
     DevBuf& buf(const char* name) {
-        if (!arena) return bufs[name];
-        DevBuf& b = abufs[name];
+        DevBuf& b = arena ? abufs[name] : bufs[name];
         b.arena = arena;
+        b.ctx = this;
         return b;
     }
     int fail(int code, const char* fmt, ...) {
@@ -427,6 +412,45 @@ struct eik_ctx {
         return code;
     }
 };
+
+namespace eik {
+// Device memory of a context's pools.  EIK_POOL_LIMIT (test hook): the most bytes that a context and its
+// peer may hold, a device with that little memory.
+inline bool pool_alloc(eik_ctx* ctx, void** p, size_t n) {
+    std::atomic<int64_t>& held = (ctx->owner ? ctx->owner : ctx)->pooled;
+    const char* e = getenv("EIK_POOL_LIMIT");
+    if ((held += (int64_t)n) <= (e ? (int64_t)atoll(e) : INT64_MAX) && hipMalloc(p, n) == hipSuccess) return true;
+    held -= (int64_t)n;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
+inline void pool_free(eik_ctx* ctx, void* p, size_t n) {
+    (void)hipFree(p);
+    (ctx->owner ? ctx->owner : ctx)->pooled -= (int64_t)n;
+}
+// Releases the march's buffers, which no call depends on; false if there are none or a march is using them.
+bool march_release(eik_ctx* ctx);
+}  // namespace eik
+
+int DevBuf::ensure(size_t n) {
+    if (n <= cap && p) return 0;
+    const size_t want = n ? n : 16;
+    if (arena) {
+        p = arena->carve(want);
+        cap = p ? want : 0;
+        return p ? 0 : -1;
+    }
+    release();
+    if (!eik::pool_alloc(ctx, &p, want) && !(eik::march_release(ctx) && eik::pool_alloc(ctx, &p, want))) return -1;
+    cap = want;
+    return 0;
+}
+void DevBuf::release() {
+    if (p && !arena) eik::pool_free(ctx, p, cap);
+    p = nullptr;
+    cap = 0;
+}
 
 namespace eik {
 // device bytes a context's reusable pools hold (they grow to the largest call seen and are kept)
@@ -612,7 +636,7 @@ struct GridSet {
     int64_t nsrc;
 };
 int64_t march_request_bytes(const std::vector<GridSet>& sets, const eik_params& P);
-// Device buffers for marches of these sizes; false if they do not fit.
+// Device buffers for marches of these sizes (march_live from then on); false if they do not fit.
 bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst);
 constexpr int kMarchAgain = 1000;  // march_run: a list was too short (list_cap), or the limit was reached (march_ctl)
 MarchCtl march_ctl(const std::vector<InstDev>& coarse, const std::vector<InstDev>& fine);
@@ -623,6 +647,14 @@ double mix_settle();
 // near: some instance has an FP64 region (unrefined mixed solve; InstDev::xlo/xhi)
 int fim_run(eik_ctx* ctx, int nd, int prec, int kind, const InstDev* d_inst, int ninst, int64_t ntiles,
             const TTPools& pools, const void* slowpool, bool exact, bool near, FimStats* fs);
+
+// A call on a context and, if it is split, its peer: when it ends, march buffers of more than a sixteenth of
+// the device's memory are given back.
+struct MarchScope {
+    eik_ctx* c;
+    explicit MarchScope(eik_ctx* ctx);
+    ~MarchScope();
+};
 
 // no-allocation scratch (eik_noalloc.hip): resolve this device's copy once (context creation)
 void scratch_setup(int device);

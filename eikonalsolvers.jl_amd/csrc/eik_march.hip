@@ -1070,13 +1070,42 @@ bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) 
     for (int k = 0; k < kMarchBufs; k++)
         if (ctx->buf(kMarchBuf[k]).cap < need[k]) grow += (int64_t)(need[k] - ctx->buf(kMarchBuf[k]).cap);
     if (ctx->march_limit >= 0 && grow > ctx->march_limit) return false;
+    if (*std::max_element(need, need + kMarchBufs) == 0) return true;
+    ctx->march_live = true;  // (no buffer of its own is released for another)
     for (int k = 0; k < kMarchBufs; k++)
         if (need[k] && ctx->buf(kMarchBuf[k]).ensure(need[k])) {
-            (void)hipGetLastError();
-            for (const char* b : kMarchBuf) ctx->buf(b).release();
+            ctx->march_live = false;
+            (void)march_release(ctx);
             return false;
         }
+    ctx->march_used = true;
     return true;
+}
+
+static int64_t march_held(eik_ctx* ctx) {
+    int64_t b = 0;
+    for (const char* k : kMarchBuf) b += (int64_t)ctx->buf(k).cap;
+    return b;
+}
+
+bool march_release(eik_ctx* ctx) {
+    if (ctx->march_live || ctx->arena || march_held(ctx) == 0) return false;
+    if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    for (const char* b : kMarchBuf) ctx->buf(b).release();
+    return true;
+}
+
+MarchScope::MarchScope(eik_ctx* ctx) : c(ctx) {
+    c->march_used = march_held(c) > 0;
+    if (c->peer) c->peer->march_used = march_held(c->peer) > 0;
+}
+
+MarchScope::~MarchScope() {
+    size_t fr = 0, tot = 0;
+    const int64_t held = march_held(c) + (c->peer ? march_held(c->peer) : 0);
+    if (held < ((int64_t)1 << 30) || hipMemGetInfo(&fr, &tot) != hipSuccess || held <= (int64_t)(tot / 16)) return;
+    (void)march_release(c);
+    if (c->peer) (void)march_release(c->peer);
 }
 
 // The limit lies far above what a converging march needs (measured: up to 9 rounds per grid node along
