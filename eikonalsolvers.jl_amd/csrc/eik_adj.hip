@@ -990,6 +990,7 @@ static int adj_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, int64_t nti
         }
         CK(hipMemcpyAsync(h_cnt, d_cnt, kAdjWords * sizeof(unsigned), hipMemcpyDeviceToHost, st));
         CK(hipStreamSynchronize(st));
+        march_give_back(ctx);  // (on a server, for a request that came during the adjoint)
         if (h_cnt[kAdjSlots + (int)((round - 1) & 1)] == 0u) break;
         if (round > 50000) return ctx->fail(EIK_ENOCONV, "adjoint solve did not converge");
     }

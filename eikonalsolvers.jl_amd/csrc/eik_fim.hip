@@ -1297,6 +1297,7 @@ int forward_solve(eik_ctx* ctx, const std::vector<FwdGroup>& G, int prec, const 
     int rc = forward_solve_once(ctx, G, prec, P);
     const bool marched = ctx->march_live;
     ctx->march_live = false;
+    march_give_back(ctx);
     if (rc != kMarchAgain && !(rc == EIK_ENOMEM && marched && march_release(ctx))) return rc;
     if (getenv("EIK_VERBOSE")) fprintf(stderr, "libeik: march stopped short, solving with tiles\n");
     const bool only = ctx->tiles_only;

@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <string>
@@ -385,7 +386,11 @@ struct eik_ctx {
     eik_ctx* owner = nullptr;  // set on a peer: the context it belongs to (whose tbase it shares)
     bool split = true;         // large calls may split their sources with the peer
     bool in_split = false;     // the current call is split (set on the context and its peer)
-    int64_t march_limit = -1;  // bytes the march's buffers may grow by in this call (-1: no limit)
+    int64_t march_limit = -1;  // bytes the march's buffers may hold in this call (-1: no limit)
+    // set by another thread: the march's buffers are wanted back as soon as the running call's march has ended
+    // (march_give_back, which reports it through march_yielded)
+    std::atomic<bool> march_yield{false};
+    std::function<void()> march_yielded;
     bool march_live = false;   // a march has its buffers (forward_solve)
     bool march_used = false;   // march buffers have been held in this call (MarchScope)
     std::atomic<int64_t> pooled{0};  // bytes of its own and its peer's buffers (kept by the owner)
@@ -431,6 +436,14 @@ inline void pool_free(eik_ctx* ctx, void* p, size_t n) {
 }
 // Releases the march's buffers, which no call depends on; false if there are none or a march is using them.
 bool march_release(eik_ctx* ctx);
+int64_t march_held(eik_ctx* ctx);  // their bytes
+// ... when they are wanted back (march_yield)
+inline void march_give_back(eik_ctx* ctx) {
+    if (!ctx->march_yield.load(std::memory_order_relaxed) || ctx->march_live) return;
+    ctx->march_yield = false;
+    (void)march_release(ctx);
+    ctx->march_yielded();
+}
 }  // namespace eik
 
 int DevBuf::ensure(size_t n) {

@@ -1066,10 +1066,15 @@ bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) 
         for (size_t n : need) sum += n + 256;
         if (sum > ctx->arena->spare) return false;
     }
-    int64_t grow = 0;
-    for (int k = 0; k < kMarchBufs; k++)
-        if (ctx->buf(kMarchBuf[k]).cap < need[k]) grow += (int64_t)(need[k] - ctx->buf(kMarchBuf[k]).cap);
-    if (ctx->march_limit >= 0 && grow > ctx->march_limit) return false;
+    if (ctx->march_limit >= 0) {
+        int64_t sum = 0, grown = 0;
+        for (int k = 0; k < kMarchBufs; k++) {
+            sum += (int64_t)need[k];
+            grown += (int64_t)std::max(need[k], ctx->buf(kMarchBuf[k]).cap);
+        }
+        if (sum > ctx->march_limit) return false;
+        if (grown > ctx->march_limit) (void)march_release(ctx);
+    }
     if (*std::max_element(need, need + kMarchBufs) == 0) return true;
     ctx->march_live = true;  // (no buffer of its own is released for another)
     for (int k = 0; k < kMarchBufs; k++)
@@ -1082,7 +1087,7 @@ bool march_reserve(eik_ctx* ctx, const MarchSize* sizes, int nsizes, int ninst) 
     return true;
 }
 
-static int64_t march_held(eik_ctx* ctx) {
+int64_t march_held(eik_ctx* ctx) {
     int64_t b = 0;
     for (const char* k : kMarchBuf) b += (int64_t)ctx->buf(k).cap;
     return b;

@@ -21,6 +21,11 @@
 // less a reserve.  When the sum does not fit but would without the pools that idle slots keep,
 // those pools are released first.  A request larger than the whole budget fails at once with
 // EIK_ENOMEM, and a call that still runs out of device memory is retried once on released pools.
+//
+// The march's buffers, which a call can do without, are counted beside that: a call is granted them from
+// what is left when every idle slot could take a request of the same size, so no request is refused
+// for them, and none waits longer than a march: a waiting request that would fit without a running
+// call's march has that call give the buffers back when its march ends.  Kept ones are the first to go.
 #include <chrono>
 #include <condition_variable>
 #include <cstring>
@@ -69,8 +74,10 @@ struct eik_server {
     int64_t reserve = 0;
     double bypass_ms = kMaxBypassMs;
     std::vector<eik_ctx*> slots;
-    std::vector<int64_t> held;  // per slot: device bytes its pools keep
-    std::vector<int64_t> run;   // per slot: working set of the request it runs (0: idle)
+    std::vector<int64_t> held;   // per slot: device bytes its pools keep, without the march's buffers
+    std::vector<int64_t> mheld;  // per idle slot: bytes of march buffers it keeps
+    std::vector<int64_t> run;    // per slot: working set of the request it runs (0: idle)
+    std::vector<int64_t> mrun;   // per slot: bytes of march buffers granted to that request
     std::vector<std::thread> workers;
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
@@ -141,11 +148,12 @@ static void run_request(eik_server* S, eik_ctx* ctx, Req& q) {
 }
 
 // What the slots would hold with a request of b bytes on slot `slot`: every other slot the
-// larger of its retained pools and its running request's working set, this slot the same.
+// larger of its retained pools and its running request's working set, and the march buffers it keeps or
+// has been granted; this slot its pools alone (its march buffers are granted anew, or released).
 static int64_t footprint_with(const eik_server* S, int slot, int64_t b) {
     int64_t t = 0;
     for (size_t o = 0; o < S->slots.size(); o++)
-        t += (int)o == slot ? std::max(S->held[o], b) : std::max(S->held[o], S->run[o]);
+        t += (int)o == slot ? std::max(S->held[o], b) : std::max(S->held[o], S->run[o]) + (S->run[o] ? S->mrun[o] : S->mheld[o]);
     return t;
 }
 
@@ -157,6 +165,7 @@ static int64_t budget_now(eik_server* S) {
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) return S->budget_now;  // keep the last reading
     int64_t h = 0;
     for (int64_t x : S->held) h += x;
+    for (int64_t x : S->mheld) h += x;
     return S->budget_now = std::max<int64_t>(0, (int64_t)fr + h - S->reserve);
 }
 
@@ -174,29 +183,67 @@ static void reject(eik_server* S, Req& q, int64_t B) {
     S->cv_done.notify_all();
 }
 
-// Whether a request of b bytes can run on idle slot `slot` within budget B; releases the pools
-// of idle slots when that makes the room.  Called with the server lock held (an idle slot's
-// context is then in no call).  A release waits for the device (hipFree synchronises), so the
+// Whether a request of b bytes can run on idle slot `slot` within budget B; releases the march buffers
+// and then the pools of idle slots when that makes the room.  Called with the server lock held (an idle
+// slot's context is then in no call).  A release waits for the device (hipFree synchronises), so the
 // other slots' running calls finish first; it happens only when the budget binds.
 static bool admit(eik_server* S, int slot, int64_t b, int64_t B) {
     if (footprint_with(S, slot, b) <= B) return true;
-    int64_t floor = b;  // the footprint with every idle slot's pools released
+    int64_t floor = b, marches = 0;  // the footprint with every idle slot's buffers released
     for (size_t o = 0; o < S->slots.size(); o++)
-        if ((int)o != slot && S->run[o]) floor += std::max(S->held[o], S->run[o]);
+        if ((int)o != slot && S->run[o]) {
+            floor += std::max(S->held[o], S->run[o]);
+            marches += S->mrun[o];
+        }
     if (floor > B) return false;  // running work holds the room: wait for it
+    if (floor + marches > B) {    // only its marches do: until they end
+        for (size_t o = 0; o < S->slots.size(); o++)
+            if ((int)o != slot && S->mrun[o]) S->slots[o]->march_yield = true;
+        return false;
+    }
+    for (size_t o = 0; o < S->slots.size() && footprint_with(S, slot, b) > B; o++) {
+        if ((int)o == slot || S->run[o] || S->mheld[o] == 0) continue;
+        (void)march_release(S->slots[o]);
+        S->mheld[o] = 0;
+    }
     for (size_t k = 0; k <= S->slots.size() && footprint_with(S, slot, b) > B; k++) {
         const size_t o = k == 0 ? (size_t)slot : k - 1;  // this slot's own pools first
         if (S->run[o] || S->held[o] == 0) continue;
         ctx_trim(S->slots[o]);
-        S->held[o] = 0;
+        S->held[o] = S->mheld[o] = 0;
         S->trims++;
     }
     return footprint_with(S, slot, b) <= B;
 }
 
+// Bytes of march buffers granted to a request of `bytes` that slot `slot` is about to run: all it wants (and
+// those the slot keeps already, if they fit), or none.  What is left of the budget is first kept for the
+// idle slots: for each a request as large as this one, or as the largest queued one that fits.  Called
+// with the server lock held.
+static int64_t march_grant(const eik_server* S, int slot, int64_t bytes, int64_t want) {
+    const int64_t room = S->budget_now - footprint_with(S, slot, bytes);
+    int64_t next = bytes, keep = 0;
+    for (int64_t k : S->queue) {
+        const int64_t b = S->reqs.at(k).bytes;
+        if (b <= room) next = std::max(next, b);
+    }
+    for (size_t o = 0; o < S->slots.size(); o++)
+        if ((int)o != slot && !S->run[o]) keep += std::max<int64_t>(0, next - S->held[o] - S->mheld[o]);
+    if (want > room - keep) return 0;
+    return S->mheld[slot] <= room - keep ? std::max(want, S->mheld[slot]) : want;
+}
+
 static void worker(eik_server* S, int slot) {
     eik_ctx* ctx = S->slots[slot];
     (void)hipSetDevice(S->device);
+    ctx->march_yielded = [S, slot, ctx] {  // (called without the server lock, by this thread)
+        ctx->march_limit = 0;
+        {
+            std::lock_guard<std::mutex> g(S->mu);
+            S->mrun[slot] = 0;
+        }
+        S->cv_work.notify_all();
+    };
     std::unique_lock<std::mutex> lk(S->mu);
     for (;;) {
         int64_t id = -1;
@@ -242,18 +289,17 @@ static void worker(eik_server* S, int slot) {
                 ++it;
             }
         }
-        // what the budget leaves beside the requests goes to the march's buffers, if they fit: with
-        // less the call runs on the tile solver, so no request is held or refused for them
         std::vector<GridSet> sets;
         for (int64_t k : ids) sets.push_back(GridSet{&S->reqs[k].r.model->g, S->reqs[k].r.nsrc});
-        int64_t extra = march_request_bytes(sets, S->reqs[id].r.params);
-        const int64_t room = S->budget_now - footprint_with(S, slot, std::max(bytes, S->held[slot]));
-        if (extra > room) extra = 0;
-        ctx->march_limit = extra;
+        const int64_t grant = march_grant(S, slot, bytes, march_request_bytes(sets, S->reqs[id].r.params));
+        ctx->march_limit = grant;
+        ctx->march_yield = false;
+        const bool drop = S->mheld[slot] > grant;
+        S->mrun[slot] = grant;
+        S->mheld[slot] = 0;
         int busy = 0;
         for (size_t o = 0; o < S->slots.size(); o++) busy += (int)o != slot && S->run[o] > 0;
         ctx->shared_device = busy >= kBusySlots;
-        bytes += extra;
         S->inflight_bytes += bytes;
         S->run[slot] = bytes;
         const Clock::time_point t0 = Clock::now();
@@ -268,6 +314,7 @@ static void worker(eik_server* S, int slot) {
         std::vector<Req*> qs;
         for (int64_t k : ids) qs.push_back(&S->reqs[k]);  // std::map nodes stay put while unlocked
         lk.unlock();
+        if (drop) (void)march_release(ctx);
         if (qs.size() == 1) {
             run_request(S, ctx, *qs[0]);
         } else {
@@ -283,10 +330,11 @@ static void worker(eik_server* S, int slot) {
                 for (Req* q : qs) run_request(S, ctx, *q);  // each request gets its own outcome
             }
         }
-        const int64_t now_held = ctx_pool_bytes(ctx);
+        const int64_t now_march = march_held(ctx), now_held = ctx_pool_bytes(ctx) - now_march;
         lk.lock();
         S->held[slot] = now_held;
-        S->run[slot] = 0;
+        S->mheld[slot] = now_march;
+        S->run[slot] = S->mrun[slot] = 0;
         const Clock::time_point t1 = Clock::now();
         for (Req* q : qs) {
             q->t_end = t1;
@@ -310,8 +358,7 @@ int eik_server_create(int32_t device, int32_t nslots, int64_t mem_budget, eik_se
     eik_server* S = new eik_server();
     S->device = device;
     S->budget = mem_budget;
-    S->held.assign((size_t)nslots, 0);
-    S->run.assign((size_t)nslots, 0);
+    for (std::vector<int64_t>* v : {&S->held, &S->mheld, &S->run, &S->mrun}) v->assign((size_t)nslots, 0);
     if (const char* e = getenv("EIK_SERVER_BYPASS_MS")) S->bypass_ms = std::max(0.0, atof(e));
     for (int i = 0; i < nslots; i++) {
         eik_ctx* c = nullptr;
@@ -422,6 +469,7 @@ int eik_server_stats(eik_server* S, int64_t* out, int32_t nout) {
     int64_t running = 0, held = 0;
     for (auto& kv : S->reqs) running += kv.second.started && !kv.second.done;
     for (int64_t x : S->held) held += x;
+    for (int64_t x : S->mheld) held += x;
     const int64_t v[10] = {(int64_t)S->queue.size(), running, S->inflight_bytes, S->budget_now, S->nbatches,
                            S->nbatched, held, S->rejected, S->trims, S->retries};
     for (int i = 0; i < nout && i < 10; i++) out[i] = v[i];
