@@ -1448,15 +1448,6 @@ static int forward_solve_once(eik_ctx* ctx, const std::vector<FwdGroup>& G, int 
     // full, a server near its budget).
     MarchSize msz[2] = {march_size(nd, kind, prec, ntiles_c, stiles_c, most_c, (int)nsrc, (int)G.size()),
                         march_size(nd, kind, EIK_PREC_FP64, ntiles_f, ntiles_f, most_f, (int)nsrc, (int)nsrc)};
-    // On a device that other calls keep busy, large sets leave the whole-device rounds to the tiles.  A call
-    // with the device to itself is faster with them (149^3 x 27 gradient 145 ms, tiles 168; 108^3 x 24
-    // 44, tiles 71), but rounds that fill it gain nothing from one another, where the tiles' longer rounds
-    // overlap: 32 requests up to 157^3 on four slots, all at once, 1.6-1.9 s with marches throughout, 1.1 s
-    // with this rule or on tiles alone.  Small sets do overlap (a queue of requests up to 64^3: 23 ms, tiles
-    // 46-50; lines at 4 M, 8 M and 16 M nodes: 31 / 23 / 23.7).
-    constexpr int64_t kFillNodes = 8000000;
-    for (MarchSize& z : msz)
-        if (ctx->shared_device && z.mode == kMarchDevice && z.ntiles * 64 >= kFillNodes) z.mode = kMarchNone;
     const bool fits = march_reserve(ctx, msz, P->refinearoundsrc ? 2 : 1, (int)nsrc);
     const bool march = fits && msz[0].mode != kMarchNone;                           // the grids
     const bool march_f = fits && P->refinearoundsrc && msz[1].mode != kMarchNone;   // the refined boxes

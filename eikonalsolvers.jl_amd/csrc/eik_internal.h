@@ -394,7 +394,6 @@ struct eik_ctx {
     bool march_live = false;   // a march has its buffers (forward_solve)
     bool march_used = false;   // march buffers have been held in this call (MarchScope)
     std::atomic<int64_t> pooled{0};  // bytes of its own and its peer's buffers (kept by the owner)
-    bool shared_device = false;  // other calls keep the device busy beside this one (see forward_solve)
     bool tiles_only = false;   // the tile solver instead of a march (see forward_solve)
     int xcap = 1;  // capacity per source of the transferred-point list
     std::mutex mu;

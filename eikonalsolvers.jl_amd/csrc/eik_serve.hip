@@ -114,12 +114,6 @@ static int64_t request_bytes(const eik_request& r) {
     return b + (4 << 20);
 }
 
-// With this many other slots running, the device counts as busy beside a request (its large grids are
-// then solved by tiles, see forward_solve).  Four slots, requests arriving at half the saturated rate: p50
-// 41 ms with marches throughout, 47-50 so, 69-97 on tiles alone.  (From two others on: p50 of a full queue
-// 500 ms rather than 290-375.)
-constexpr int kBusySlots = 3;
-
 static int call_request(eik_ctx* ctx, const eik_request& r) {
     if (r.type == EIK_REQ_TRAVELTIME)
         return eik_traveltime(ctx, r.model, r.nsrc, r.coordsrc, r.rec_off, r.coordrec, &r.params, r.ttpicks, nullptr);
@@ -297,9 +291,6 @@ static void worker(eik_server* S, int slot) {
         const bool drop = S->mheld[slot] > grant;
         S->mrun[slot] = grant;
         S->mheld[slot] = 0;
-        int busy = 0;
-        for (size_t o = 0; o < S->slots.size(); o++) busy += (int)o != slot && S->run[o] > 0;
-        ctx->shared_device = busy >= kBusySlots;
         S->inflight_bytes += bytes;
         S->run[slot] = bytes;
         const Clock::time_point t0 = Clock::now();
