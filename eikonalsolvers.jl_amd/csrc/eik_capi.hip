@@ -318,9 +318,15 @@ int eik_model_create(eik_ctx* ctx, const eik_grid* grid, const double* vel, eik_
     for (int d = 0; d < grid->ndim; d++) M->N *= grid->n[d];
     for (int d = grid->ndim; d < 3; d++) M->g.n[d] = 1;
     (void)hipSetDevice(ctx->device);
-    if (hipMalloc(&M->d_vel, M->N * sizeof(double)) != hipSuccess ||
-        hipMalloc(&M->d_slow64, M->N * sizeof(double)) != hipSuccess ||
-        hipMalloc(&M->d_slow32, M->N * sizeof(float)) != hipSuccess) {
+    // (march buffers that the context and its peer keep from earlier calls give way to a model)
+    const auto take = [&](void** p, size_t n) {
+        if (hipMalloc(p, n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        const bool a = march_release(ctx), b = ctx->peer && march_release(ctx->peer);
+        return (a || b) && hipMalloc(p, n) == hipSuccess;
+    };
+    if (!take((void**)&M->d_vel, M->N * sizeof(double)) || !take((void**)&M->d_slow64, M->N * sizeof(double)) ||
+        !take((void**)&M->d_slow32, M->N * sizeof(float))) {
         eik_model_destroy(M);
         return ctx->fail(EIK_ENOMEM, "out of device memory (model)");
     }
