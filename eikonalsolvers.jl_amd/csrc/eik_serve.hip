@@ -210,10 +210,10 @@ static bool admit(eik_server* S, int slot, int64_t b, int64_t B) {
     return footprint_with(S, slot, b) <= B;
 }
 
-// Bytes of march buffers granted to a request of `bytes` that slot `slot` is about to run: all it wants (and
-// those the slot keeps already, if they fit), or none.  What is left of the budget is first kept for the
-// idle slots: for each a request as large as this one, or as the largest queued one that fits.  Called
-// with the server lock held.
+// Bytes of march buffers granted to a request of `bytes` that slot `slot` is about to run: all it wants beside
+// those the slot keeps (which another shape of request needs larger one by one), all it wants in their
+// place, or none.  What is left of the budget is first kept for the idle slots: for each a request as large as
+// this one, or as the largest queued one that fits.  Called with the server lock held.
 static int64_t march_grant(const eik_server* S, int slot, int64_t bytes, int64_t want) {
     const int64_t room = S->budget_now - footprint_with(S, slot, bytes);
     int64_t next = bytes, keep = 0;
@@ -223,8 +223,8 @@ static int64_t march_grant(const eik_server* S, int slot, int64_t bytes, int64_t
     }
     for (size_t o = 0; o < S->slots.size(); o++)
         if ((int)o != slot && !S->run[o]) keep += std::max<int64_t>(0, next - S->held[o] - S->mheld[o]);
-    if (want > room - keep) return 0;
-    return S->mheld[slot] <= room - keep ? std::max(want, S->mheld[slot]) : want;
+    if (want + S->mheld[slot] <= room - keep) return want + S->mheld[slot];
+    return want <= room - keep ? want : 0;
 }
 
 static void worker(eik_server* S, int slot) {
