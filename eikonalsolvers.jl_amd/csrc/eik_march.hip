@@ -41,8 +41,8 @@ namespace eik {
 
 constexpr unsigned kIdle = 0x7f800000u;  // P of a node that is not pending: +inf
 
-// A list entry: node, the stencil position that held it up when last looked at (kNoHint: none), and
-// kOnce once the entry is known to be its node's only one.
+// A list entry: node, and either kOnce, once the entry is known to be its node's only one, with the stencil
+// position that held it up when last looked at (kNoHint: none), or in a device round its waker's tag.
 constexpr unsigned kNodeBits = 27, kNodeMask = (1u << kNodeBits) - 1u;
 constexpr unsigned kHintShift = kNodeBits, kNoHint = 15u, kOnce = 0x80000000u;
 constexpr unsigned kNoEntry = 0xffffffffu;  // (no march has kNodeMask nodes)
@@ -115,8 +115,8 @@ struct MarchPools {
     T* tt;
     const T* slow;    // per model: InstDev::ms_off
     unsigned* p[3];   // pending values
-    unsigned* own;    // list position of a node's newest entry
-    unsigned* less;   // a listed node's pending value lowered by a later wake (k_march_round)
+    unsigned* own;    // list position of a node's newest entry (a workgroup per instance)
+    unsigned* less;   // a listed node's pending value lowered by a later wake (device rounds)
     unsigned* lists;  // two lists per instance (list_start)
 };
 
@@ -162,6 +162,13 @@ __device__ __forceinline__ bool quiet_change(T v0, T k0, T v1, T k1, T settle) {
 // The pending value of a woken node, as bits: never 0 (may_run steps it down by one), and never an
 // idle node's, whatever the expected value (times beyond the float range: its largest number).
 __device__ __forceinline__ unsigned pend_bits(float p) { return min(max(__float_as_uint(p), 1u), kIdle - 1u); }
+
+// The same in a device round, with the stencil position k of the woken node as seen from the node that wakes
+// it in the low bits (20 bits of mantissa are left for the order).  No two nodes of a round wake a node with
+// the same k, so the minimum that the node ends up with names one of them.
+constexpr unsigned kTagMask = 15u;
+__device__ __forceinline__ unsigned wake_tag(int k) { return (unsigned)k + 1u; }
+__device__ __forceinline__ unsigned pend_tagged(float p, int k) { return (pend_bits(p) & ~kTagMask) | wake_tag(k); }
 
 // Replays node l (on: this lane has one) and writes it if it changed; returns whether it did.
 // p: the round's pending values (only read here).  wake(k, w, q, idle, pq, p): if w, neighbour q (the
@@ -388,15 +395,16 @@ __device__ __forceinline__ unsigned lane_rank(unsigned long long m) {
 // For phases that exchange nothing through memory.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Listing.  Several nodes of a round may wake the same idle node; each lists it and writes its own
-// list position into the node's `own` word, and the next selection drops the entries that the word
-// does not name.  No atomic's return value is waited for.  Where the writers are blocks of several XCDs
-// the word is written by an atomic: after two plain stores from two XCDs in one launch each XCD went on
-// reading its own in the next, so that both entries stood, and one of them stayed listed for good when
-// the node had run.
+// Listing.  Several nodes of a round may wake the same idle node, and each lists it; the next selection drops
+// all entries but one, without waiting for an atomic's return value.  In a workgroup each writes its list
+// position into the node's `own` word, and the entry that the word names stands.  In a device round, whose
+// blocks run on several XCDs, that would be a race on memory (after plain stores from two XCDs in one launch
+// each went on reading its own in the next: both entries stood, and one was left listed for good when the
+// node had run), so the entry carries its waker's tag, and the one stands whose tag the node's pending value
+// carries (pend_tagged).
 
 // The neighbours of the init nodes (values in the x-fastest pool) are pending with their smallest init
-// neighbour's value: add(q, p) for each of them, by the threads of one block.  The init nodes'
+// neighbour's value: add(q, p, k) for each of them, k its position from that neighbour, by the threads of one block.  The init nodes'
 // values go to the bricked pool first.
 template <int ND, typename T, class Add>
 __device__ __forceinline__ void seed_march(const InstDev& I, const GridView<ND, T>& G, const T* tt_lin, const SrcPt* seeds, int ns,
@@ -422,7 +430,7 @@ __device__ __forceinline__ void seed_march(const InstDev& I, const GridView<ND, 
         g[2] += ax == 2 ? sh : 0;
         if (g[0] < 0 || g[0] >= G.n[0] || g[1] < 0 || g[1] >= G.n[1] || g[2] < 0 || g[2] >= G.n[2]) continue;
         const unsigned q = G.index(g);
-        if (!signbit(G.tt[q])) add(q, pend_bits((float)fabs(tt_lin[l])));
+        if (!signbit(G.tt[q])) add(q, (float)fabs(tt_lin[l]), k);
     }
 }
 
@@ -467,8 +475,8 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
     }
     if (tid < 2) s_nrun[tid] = 0u;
     __syncthreads();
-    seed_march<ND, T>(I, G, (const T*)pools.tt + I.tt_off, seeds + (int64_t)blockIdx.x * cap, nseed[blockIdx.x], [&](unsigned q, unsigned p) {
-        const unsigned at = atomicAdd(&s_cnt[0], 1u);
+    seed_march<ND, T>(I, G, (const T*)pools.tt + I.tt_off, seeds + (int64_t)blockIdx.x * cap, nseed[blockIdx.x], [&](unsigned q, float pf, int) {
+        const unsigned at = atomicAdd(&s_cnt[0], 1u), p = pend_bits(pf);
         lower(q, p);
         atomicMin(&s_min[0], p);
         own[q] = at;
@@ -633,7 +641,6 @@ __global__ void __launch_bounds__(256) k_march_seed(const InstDev* __restrict__ 
     const unsigned scap = min(seg_cap(64u * (unsigned)(I.t[0] * I.t[1] * I.t[2]), blocks), S.limit);
     unsigned* const list = inst_lists(M, I, in, blocks);
     unsigned* const pend = M.p[0] + I.tile_base * 64;
-    unsigned* const own = M.own + I.tile_base * 64;
     if (threadIdx.x == 0) {
         s_n = 0u;
         s_low = kIdle;
@@ -643,12 +650,11 @@ __global__ void __launch_bounds__(256) k_march_seed(const InstDev* __restrict__ 
         S.stat[2 * (in * blocks + b)] = S.stat[2 * (in * blocks + b) + 1] = 0u;
     }
     __syncthreads();
-    seed_march<ND, T>(I, G, (const T*)pools.tt + I.tt_off, seeds + (int64_t)in * cap, nseed[in], [&](unsigned q, unsigned p) {
-        const unsigned at = atomicAdd(&s_n, 1u);
+    seed_march<ND, T>(I, G, (const T*)pools.tt + I.tt_off, seeds + (int64_t)in * cap, nseed[in], [&](unsigned q, float pf, int k) {
+        const unsigned at = atomicAdd(&s_n, 1u), p = pend_tagged(pf, k);
         atomicMin(&pend[q], p);
         atomicMin(&s_low, p);
-        own[q] = at;
-        if (at < scap) list[at] = q | kNoHint << kHintShift;
+        if (at < scap) list[at] = q | wake_tag(k) << kHintShift;
     });
     __syncthreads();
     if (threadIdx.x == 0 && s_n > scap) atomicOr(&counters[3], kOverflow);
@@ -690,7 +696,6 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
     const unsigned* const p = M.p[slot] + I.tile_base * 64;
     unsigned* const pn = M.p[nslot] + I.tile_base * 64;
     unsigned* const pr = M.p[rslot] + I.tile_base * 64;
-    unsigned* const own = M.own + I.tile_base * 64;
     unsigned* const less = M.less + I.tile_base * 64;
     const unsigned scap = min(seg_cap(nodes, nblk), S.limit), half = scap * nblk;  // a list: nblk segments
     const unsigned* const from = inst_lists(M, I, in, (int)nblk) + (par ? half : 0u);
@@ -737,7 +742,7 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             s_nfresh = 0u;
         }
         lds_barrier();  // also: every thread has read the run list of the last round
-        unsigned e[kRoundPer], pv[kRoundPer], pb[kRoundPer], pos[kRoundPer];
+        unsigned e[kRoundPer], pv[kRoundPer], pb[kRoundPer];
 #pragma unroll
         for (int u = 0; u < kRoundPer; u++) {
             // entry i lies in the segment whose end is the first beyond i
@@ -745,19 +750,17 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             unsigned s = (unsigned)__popcll(__ballot(end <= i0));
             if (i < hi)
                 while (s_end[wave][s] <= i) s++;
-            pos[u] = s * scap + (i - (s ? s_end[wave][s - 1] : 0u));
-            e[u] = i < hi ? from[pos[u]] : kNoEntry;
+            e[u] = i < hi ? from[s * scap + (i - (s ? s_end[wave][s - 1] : 0u))] : kNoEntry;
         }
         if (base == lo) clear_ran();
         // own value, that of the node that held it up before, and a lowered one, in one round trip
-        unsigned ls[kRoundPer], ow[kRoundPer];
+        unsigned ls[kRoundPer];
 #pragma unroll
         for (int u = 0; u < kRoundPer; u++) {
             const bool have = e[u] != kNoEntry;
-            const unsigned l = have ? e[u] & kNodeMask : 0u, h = (e[u] >> kHintShift) & 15u;
+            const unsigned l = have ? e[u] & kNodeMask : 0u, h = (e[u] & kOnce) ? (e[u] >> kHintShift) & 15u : kNoHint;
             pv[u] = at<ND>(p, l);
             pb[u] = at<ND>(p, hints && have && h != kNoHint ? hint_index<ND, T>(G, l, h) : l);
-            ow[u] = at<ND>(own, have && !(e[u] & kOnce) ? l : 0u);
             ls[u] = at<ND>(less, l);
         }
         // the other stencil positions of the entries that are not held up still, in another
@@ -765,8 +768,8 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         bool run[kRoundPer];
 #pragma unroll
         for (int u = 0; u < kRoundPer; u++) {
-            const unsigned h = (e[u] >> kHintShift) & 15u;
-            if (e[u] != kNoEntry && !(e[u] & kOnce) && ow[u] != pos[u]) e[u] = kNoEntry;
+            const unsigned t = (e[u] >> kHintShift) & 15u, h = (e[u] & kOnce) ? t : kNoHint;
+            if (e[u] != kNoEntry && !(e[u] & kOnce) && t != (pv[u] & kTagMask)) e[u] = kNoEntry;
             // still held up: lower, or as low and further down
             const bool held = hints && h != kNoHint && (pb[u] < pv[u] || ((h & 1u) && pb[u] == pv[u]));
             run[u] = e[u] != kNoEntry && pv[u] <= lim && !held;
@@ -810,10 +813,8 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
         }
         lds_barrier();
         const unsigned nrun = min(s_nrun, (unsigned)kRoundRun), nkeep = s_nkeep;
-        // blocks on several XCDs may list a node in one round: an atomic (see "Listing" above)
-        const auto list_fresh = [&](unsigned j, unsigned l) {
-            if (j < scap) to[j] = l | kNoHint << kHintShift;
-            (void)__hip_atomic_exchange(&at<ND>(own, l), blk * scap + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const auto list_fresh = [&](unsigned j, unsigned e) {
+            if (j < scap) to[j] = e;
         };
         for (unsigned b = done + (unsigned)(tid & ~63); b < nrun; b += kRoundThreads) {
             const unsigned j = b + lane;
@@ -829,8 +830,8 @@ __global__ void __launch_bounds__(kRoundThreads, 2)
             bool two;
             const bool chg = relax_node<ND, T, SPH, MIX, NEAR>(
                 I, G, mcart, p, l, on, settle, &two, [&](int k, bool w, unsigned q, bool idle, unsigned pq, float pf) {
-                    who[k] = q;
-                    const unsigned pu = pend_bits(pf);
+                    who[k] = q | wake_tag(k) << kHintShift;
+                    const unsigned pu = pend_tagged(pf, k);
                     if (w && pu < pq) {
                         lowest = min(lowest, pu);
                         atomicMin(idle ? &at<ND>(pn, q) : &at<ND>(less, q), pu);
@@ -1158,8 +1159,8 @@ static int march_run_t(eik_ctx* ctx, const InstDev* d_inst, int ninst, const Mar
     const int64_t nb = sz.ntiles * 64;
     unsigned* pend = (unsigned*)ctx->buf("march_pend").p;  // march_reserve made the buffers
     MarchPools<T> M{(T*)ctx->buf("march_tt").p, (const T*)ctx->buf("march_slow").p, {pend, pend + nb, pend + 2 * nb},
-                    (unsigned*)ctx->buf("march_own").p, (unsigned*)ctx->buf("march_own").p + nb,
-                    (unsigned*)ctx->buf("march_list").p};  // (p[1], p[2] and less: device rounds alone)
+                    (unsigned*)ctx->buf("march_own").p, (unsigned*)ctx->buf("march_own").p,  // (one or the other)
+                    (unsigned*)ctx->buf("march_list").p};
     unsigned long long* d_c = (unsigned long long*)ctx->buf("march_cnt").p;
     unsigned long long* h = (unsigned long long*)ctx->h_small;
     const bool device = sz.mode == kMarchDevice;

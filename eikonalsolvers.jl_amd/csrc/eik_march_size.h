@@ -43,8 +43,8 @@ EIK_HD int64_t list_start(int64_t tile_base, int64_t in, int blocks) {
 }
 
 // Bytes of the march's buffers for ninst instances of ntiles bricks in all and stiles bricks of slowness grids:
-// values, slowness, pending values, own words (and lowered values), lists, counters and segment words, run lists.
-// In FP64 a workgroup per instance takes 26 bytes a node and 64 KB an instance, device rounds 48 and up to
+// values, slowness, pending values, own words or lowered values, lists, counters and segment words, run lists.
+// In FP64 a workgroup per instance takes 26 bytes a node and 64 KB an instance, device rounds 44 and up to
 // 2.4 MB; a slowness grid 8 bytes a node of its model.
 constexpr int kMarchBufs = 7;
 inline void march_bytes(int mode, int64_t ntiles, int64_t stiles, int ninst, size_t esz, size_t* need) {
@@ -56,7 +56,7 @@ inline void march_bytes(int mode, int64_t ntiles, int64_t stiles, int ninst, siz
     need[0] = nb * esz;
     need[1] = (size_t)stiles * 64 * esz;
     need[2] = (device ? 3 : 1) * nb * sizeof(unsigned);
-    need[3] = (device ? 2 : 1) * nb * sizeof(unsigned);
+    need[3] = nb * sizeof(unsigned);
     need[4] = (size_t)list_start(ntiles, ninst, blocks) * sizeof(unsigned);
     need[5] = 256 + (device ? (4 * kMaxBlocks + 2 * (size_t)blocks) * (size_t)ninst * sizeof(unsigned) : 0);
     need[6] = device ? (size_t)ninst * blocks * (kRoundRun + 1) * sizeof(unsigned) : 0;
