@@ -165,9 +165,11 @@ __device__ __forceinline__ unsigned pend_bits(float p) { return min(max(__float_
 
 // The same in a device round, with the stencil position k of the woken node as seen from the node that wakes
 // it in the low bits (20 bits of mantissa are left for the order).  No two nodes of a round wake a node with
-// the same k, so the minimum that the node ends up with names one of them.
+// the same k, so the minimum that the node ends up with names one of them.  Among equal values the later
+// position goes first: the other way round 3D spheres need up to 18 % more rounds (50x90x90 x 5: 352 -> 416,
+// 5.6 -> 6.4 ms).
 constexpr unsigned kTagMask = 15u;
-__device__ __forceinline__ unsigned wake_tag(int k) { return (unsigned)k + 1u; }
+__device__ __forceinline__ unsigned wake_tag(int k) { return 14u - (unsigned)k; }
 __device__ __forceinline__ unsigned pend_tagged(float p, int k) { return (pend_bits(p) & ~kTagMask) | wake_tag(k); }
 
 // Replays node l (on: this lane has one) and writes it if it changed; returns whether it did.
