@@ -393,6 +393,7 @@ struct eik_ctx {
     std::function<void()> march_yielded;
     bool march_live = false;   // a march has its buffers (forward_solve)
     bool march_used = false;   // march buffers have been held in this call (MarchScope)
+    size_t mem_total = 0;      // the device's memory (MarchScope)
     std::atomic<int64_t> pooled{0};  // bytes of its own and its peer's buffers (kept by the owner)
     bool tiles_only = false;   // the tile solver instead of a march (see forward_solve)
     int xcap = 1;  // capacity per source of the transferred-point list

@@ -1109,9 +1109,10 @@ MarchScope::MarchScope(eik_ctx* ctx) : c(ctx) {
 }
 
 MarchScope::~MarchScope() {
-    size_t fr = 0, tot = 0;
     const int64_t held = march_held(c) + (c->peer ? march_held(c->peer) : 0);
-    if (held < ((int64_t)1 << 30) || hipMemGetInfo(&fr, &tot) != hipSuccess || held <= (int64_t)(tot / 16)) return;
+    size_t fr = 0;
+    if (held < ((int64_t)1 << 30) || (!c->mem_total && hipMemGetInfo(&fr, &c->mem_total) != hipSuccess)) return;
+    if (held <= (int64_t)(c->mem_total / 16)) return;
     (void)march_release(c);
     if (c->peer) (void)march_release(c->peer);
 }
