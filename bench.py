@@ -160,7 +160,9 @@ def _roofline(prec: str, f: dict) -> dict:
     if tr is not None:
         out["traffic"] = tr["hbm_bytes_per_launch"]
         out["traffic_bytes_per_step"] = round(tr["hbm_bytes_per_launch"] * tr["launches"])
-        out["traffic_over_algorithmic"] = round(out["traffic_bytes_per_step"] / max(alg_per_launch * launches, 1.0), 3)
+        # the profiled launches include, in fp64, those of the refined boxes: so do these algorithmic bytes
+        visits = f["kernel_visits_per_step"] + (f["fine_visits_per_step"] if prec == "fp64" else 0.0)
+        out["traffic_over_algorithmic"] = round(out["traffic_bytes_per_step"] / max(visits * BYTES_PER_VISIT[prec], 1.0), 3)
         out["traffic_measured_on"] = tr.get("measured_on", "")
     return out
 
@@ -281,6 +283,7 @@ def main() -> int:
             "rounds_per_step": tot["rounds"] / args.steps,
             "launches_per_step": k_launches / args.steps,
             "kernel_visits_per_step": k_visits / args.steps,
+            "fine_visits_per_step": tot["fine_tile_activations"] * TILE_NODES_3D / args.steps,
             "kernel_all_ms_per_step": k_ms / args.steps,
             "kernel_busy_ms_per_step": k_busy / args.steps,
             "node_visits_per_step": visits / args.steps,
