@@ -1443,9 +1443,9 @@ static int forward_solve_once(eik_ctx* ctx, const std::vector<FwdGroup>& G, int 
             for (int64_t s = 0; s < nsrc; s++) finst[s].sinth = (const double*)ft.p + off[s];
         }
     }
-    // Ordered marching where its buffers fit beside the pools; the tile solver, which needs about 50
-    // bytes a node less, otherwise (a no-allocation call near its limit, a device that is nearly
-    // full, a server near its budget).
+    // Ordered marching where its buffers (26 bytes a node and 64 KB a source for one workgroup per source, 44
+    // and up to 2.4 MB for device rounds, in FP64) fit beside the pools; the tile solver otherwise (a
+    // no-allocation call near its limit, a device that is nearly full, a server near its budget).
     MarchSize msz[2] = {march_size(nd, kind, prec, ntiles_c, stiles_c, most_c, (int)nsrc, (int)G.size()),
                         march_size(nd, kind, EIK_PREC_FP64, ntiles_f, ntiles_f, most_f, (int)nsrc, (int)nsrc)};
     const bool fits = march_reserve(ctx, msz, P->refinearoundsrc ? 2 : 1, (int)nsrc);

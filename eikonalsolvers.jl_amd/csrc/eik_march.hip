@@ -20,8 +20,12 @@
 //            keys both exceed a node's key leaves its replay as it is), and of the nodes two away
 //            only those whose in-between node pops no later than they do.
 // The node with an instance's lowest P always runs, so a round always makes progress; when nothing
-// is pending every node's replay equals its value.  No read races a write in any round, so the
-// result does not depend on the schedule, and there is nothing to verify at the end.
+// is pending every node's replay equals its value, and there is nothing to verify at the end.  No read of
+// a value or key races a write: what a node's replay reads no other node of the round changes.  Pending
+// values do race (a wake may lower one while its holder reads it) and a round has room for so many nodes,
+// so the order depends on the schedule, and the result where the replay has more than one fixed point:
+// exact ties, FP32's near-ties, the roughest media.  A march can circulate where the order means
+// little; it then stops at its limit (march_ctl).
 //
 // Layout.  Values, pending values and slowness lie in bricks of 64 nodes (4x4x4, or 8x8 in 2D), so
 // that a node's stencil and the nodes around it on the front share cache lines whatever the front's
@@ -607,7 +611,7 @@ __global__ void __launch_bounds__(BT) k_march_group(const InstDev* __restrict__ 
 // launch's, so within one launch the round's pending values (buffer round % 3) and its list are only
 // read; the next round's go to buffer (round + 1) % 3 and the other list:
 //   a node that stays listed takes its value along, or a lower one that wakes have left in `less`
-//   (which only the thread that holds its entry reads);
+//   (its holder reads it while they lower it, and sees it in this round or the next);
 //   a node that runs becomes idle in the next buffer and in the third (which nobody reads or writes
 //   in this round), and in the present one a round later, when that is the third: by the block that
 //   ran it, from the list `ran` it keeps;

@@ -190,7 +190,9 @@ int eik_tracerays_max_steps(const eik_grid* grid, double steplen, int64_t* out);
  * the budget (idle slots' pools are released when that makes the room).  mem_budget > 0 fixes the
  * budget in bytes; mem_budget = 0 takes the device's free memory (read at every admission) plus
  * what the slots hold, less a reserve of max(2 GiB, 1/32 of the device).  A request whose working
- * set exceeds the whole budget fails on its own with EIK_ENOMEM (eik_wait returns it).  The arrays a
+ * set exceeds the whole budget fails on its own with EIK_ENOMEM (eik_wait returns it).  Buffers that
+ * a call can do without (the ordered march's) come out of what the budget leaves beside that, hold no
+ * request back and are given up first; they count in eik_server_stats [6].  The arrays a
  * request points to (inputs and outputs) must stay valid until eik_wait returns for it, and its
  * model must not be updated or destroyed meanwhile. */
 #define EIK_REQ_TRAVELTIME 1 /* eiktraveltime: fills ttpicks */
